@@ -1007,7 +1007,6 @@ __global__ void keys_to_tokens_kernel(const u64* keys, int R, const int32_t* bad
 // deterministic.
 // ------------------------------------------------------------------------------------------------
 constexpr int BMAX = 64;
-constexpr int KS = 64;  // keys per attention split (one round of 4 keys per 16-lane group)
 
 enum SkEpi { SK_RAW = 0, SK_PART = 1, SK_SILU = 2 };
 
@@ -1218,16 +1217,6 @@ __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tok
   }
 }
 
-// Position of sequence b, clamped into the cache (an out-of-range position sets *bad).
-__device__ __forceinline__ int seq_pos(const int32_t* positions, int b, int max_seq, int32_t* bad) {
-  const int p = positions[b];
-  if (p < 0 || p >= max_seq) {
-    if (bad) *bad = 1;
-    return p < 0 ? 0 : max_seq - 1;
-  }
-  return p;
-}
-
 // The raw Q/K/V sums of M consecutive prompt tokens of one sequence (fp32 [M][4096], or S such arrays
 // of K-range sums added in order; row m at position pos0 + m): per-head RMSNorm + RoPE on q and k,
 // q kept as a bf16 hi/lo pair [M][2048], k and v rounded to bf16 into the cache [L][8][max_seq][128].
@@ -1318,207 +1307,318 @@ __global__ void __launch_bounds__(64) silu_post_kernel(const float* part, int S,
   *reinterpret_cast<uint4*>(bl + o) = lo;
 }
 
-// Split-K attention of one sequence and K/V head over keys [KS s, KS s + KS) of [0, position]: the
-// head pair's two queries against each key (16 groups of 16 lanes, lane t holding dims 8t..8t+7,
-// keys dealt to the groups in turn, online softmax per group, /root/reference/megakernel.cu:228-370),
-// the 16 group partials merged in LDS into this split's (acc[128], m, l) per query head.
-// part: [B][8][S][2][D + 2].
-constexpr int APW = D + 2;
+// ------------------------------------------------------------------------------------------------
+// Attention of the batched decode. The keys of a step are cut into items, at most one workgroup each
+// per K/V head, by batch_plan_kernel once per step (the positions are the same in every layer).
+// ------------------------------------------------------------------------------------------------
+constexpr int KBLK = 64;  // keys per round of a workgroup: 16 groups of 16 lanes, 4 keys each
+constexpr int BU = 4;
+static_assert(KBLK == 16 * BU, "a key block is one round of loads");
+constexpr int APW = D + 4;  // floats per head of a partial: acc[128], m, l, pad (16-byte aligned)
 
+// Items that a step of B sequences may have: every sequence takes ceil(blocks / C) of them with
+// C = ceil(all blocks / PLAN_SLACK) key blocks per item, so at most PLAN_SLACK + B in all. The items
+// should be as many as run at once (battn_kernel: 3 workgroups per CU, 96 items of 8 heads) and no
+// more: measured on MI355X, us per step at 16 / 32 / 48 / 64 / 80 / 128 / 192: 13 sequences of 100 to
+// 1,900 keys (1.7B) 2,009 / 2,009 / 1,942 / 1,912 / 1,947 / 2,021 / 2,020; 64 sequences of 64 to 960
+// keys (0.6B) within 1% of each other from 16 to 128.
+constexpr int PLAN_SLACK = 64;
+__host__ __device__ inline int plan_items(int B) { return PLAN_SLACK + B; }
 
-constexpr int BU = 4;  // keys per 16-lane group and split: one round of loads
-static_assert(KS == 16 * BU, "a split is one round of loads");
+// One item: keys [k0, k1) of sequence b, split s of its ns.
+struct PlanItem {
+  int32_t seq;  // b | ns << 8 | s << 20; -1: no item
+  int32_t k0, k1;
+  uint32_t pos;  // the sequence's position; top bit: its new K/V rows may be written
+};
 
-// Group gi's keys of split s (positions k0 + gi + 16 u; past the split they re-read its last key).
-__device__ __forceinline__ void battn_load(const uint16_t* k_cache, const uint16_t* v_cache, int b, int kvh, int s,
-                                           int ctx, int L, int layer, int max_seq, uint4 (&kw)[BU],
-                                           uint4 (&vw)[BU]) {
-  const int lane = threadIdx.x & 63, gi = (threadIdx.x >> 6) * 4 + (lane >> 4), t = lane & 15;
-  const int k0 = s * KS, k1 = min(k0 + KS, ctx);
-  const size_t base = (((size_t)b * L + layer) * HKV + kvh) * max_seq * D + 8 * t;
+// The start of a batched step (one wave, lane b = sequence b): clears the greedy keys, the split
+// counters and the error flag (set again if a position is out of range: such a sequence is decoded at
+// a clamped position, its cache keeps its rows and the call reports NaN and -1), and lays out the
+// attention's items. The items go longest first, so that the CUs that finish early take short ones.
+__global__ void __launch_bounds__(64) batch_plan_kernel(const int32_t* positions, const int32_t* tokens, int vocab,
+                                                        int max_seq, int B, u64* keys, int32_t* bad, uint32_t* count,
+                                                        PlanItem* plan) {
+  const int b = threadIdx.x;
+  const bool in = b < B;
+  int p = in ? positions[b] : 0;
+  const bool off = p < 0 || p >= max_seq;
+  if (off) p = p < 0 ? 0 : max_seq - 1;
+  const bool write = in && !off && tokens[b] >= 0 && tokens[b] < vocab;
+  if (in) keys[b] = 0;
+  for (int i = b; i < B * HKV; i += 64) count[i] = 0;
+  const bool any_off = __builtin_amdgcn_ballot_w64(off) != 0;
+  if (b == 0) *bad = any_off ? 1 : 0;
+  const int nblk = in ? p / KBLK + 1 : 0;
+  int total = nblk;
 #pragma unroll
-  for (int u = 0; u < BU; ++u) {
-    const int pu = min(k0 + gi + 16 * u, k1 - 1);
-    kw[u] = *reinterpret_cast<const uint4*>(k_cache + base + (size_t)pu * D);
-    vw[u] = *reinterpret_cast<const uint4*>(v_cache + base + (size_t)pu * D);
+  for (int o = 32; o >= 1; o >>= 1) total += __shfl_xor(total, o);
+  const int C = (total + PLAN_SLACK - 1) / PLAN_SLACK;
+  int ns = (nblk + C - 1) / C;
+  const int len = ns ? (nblk + ns - 1) / ns : 0;  // key blocks per item of this sequence
+  if (len) ns = (nblk + len - 1) / len;           // no empty item
+  int first = 0, n = 0;                           // items of longer (or equal, earlier) sequences; all items
+  for (int q = 0; q < 64; ++q) {
+    const int ql = __shfl(len, q), qn = __shfl(ns, q);
+    if (ql > len || (ql == len && q < b)) first += qn;
+    n += qn;
   }
+  for (int s = 0; s < ns; ++s) {
+    PlanItem it;
+    it.seq = b | ns << 8 | s << 20;
+    it.k0 = s * len * KBLK;
+    it.k1 = min(it.k0 + len * KBLK, p + 1);
+    it.pos = (uint32_t)p | (write ? 0x80000000u : 0u);
+    plan[first + s] = it;
+  }
+  for (int i = n + b; i < plan_items(B); i += 64) plan[i].seq = -1;
 }
 
-__device__ __forceinline__ void battn_split(const float (&qa)[8], const float (&qb)[8], uint4 knew, uint4 vnew,
-                                            int pos, const uint4 (&kw)[BU], const uint4 (&vw)[BU], int b,
-                                            int kvh, int s, int ctx, float* part, int S, float (&gacc)[16][2][D],
-                                            float (&gml)[16][2][2]) {
-  const int k0 = s * KS;
-  const int k1 = min(k0 + KS, ctx);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int gi = w * 4 + (lane >> 4), t = lane & 15;
+struct BAttnArgs {
+  const float* raw;  // this layer's Q/K/V sums, fp32 [B][4096]
+  const uint16_t *q_norm, *k_norm, *cos_tab, *sin_tab;
+  uint16_t *k_cache, *v_cache;
+  int L, layer, max_seq, B;
+  const PlanItem* plan;
+  float* part;      // [item][8 heads][2][APW]: split items' unnormalised rows (acc, m, l), m in base 2
+  uint32_t* count;  // [B][8]: split items that have written theirs
+  uint16_t* out;    // the O product's skinny fragments (hi and lo)
+};
+
+// One item and K/V head per workgroup (workgroup 8 i + h: item i, head h). 16 groups of 16 lanes, lane
+// t of a group holding dims 8 t .. +7, take the item's keys in turn, 4 per round, with an online
+// softmax per group for both query heads of the pair (/root/reference/megakernel.cu:228-370), the next
+// round's K/V rows in flight while a round is computed. The new row's projections are finished here:
+// every group normalises and rotates the two queries, and the item that ends at the sequence's position
+// attends to the new K/V row from registers and writes it into the cache. The group sums are merged in
+// registers and LDS. A sequence in one item is finished at once; the items of a split one write their
+// sums through to memory and count themselves, and the last of them merges all (in split order, so the
+// result does not depend on which was last).
+//
+// Bound by the K/V stream behind ~10 us of launch, first round trips and merge. Measured on MI355X
+// (rocprofv3, per layer), against 64-key splits dealt out evenly (each split loaded, reduced over its
+// 16 groups and written as a partial in turn) and a merge kernel after them: 64 sequences of 64 to 960
+// keys (0.6B, 134 MB) 38.8 + 4.9 -> 30.0 us, the keys past the first round at 5.7 TB/s; 13 sequences of
+// 100 to 1,900 keys (1.7B, 53 MB) 18.7 + 6.5 -> 17.0 us. The non-temporal hint on the K/V rows (each is
+// read once a step) is 95 and 54 us of the step; counting the split items in and merging them costs 1.8
+// us per layer, against the merge kernel's launch.
+__global__ void __launch_bounds__(256) battn_kernel(const BAttnArgs a) {
+  __shared__ __attribute__((aligned(16))) float sacc[4][2][D];
+  __shared__ float sml[4][2][2];
+  __shared__ __attribute__((aligned(16))) float so[2][D];
+  __shared__ uint32_t arrived;
+  const PlanItem it = a.plan[blockIdx.x >> 3];
+  if (it.seq < 0) return;
+  const int kvh = blockIdx.x & 7, b = it.seq & 255, ns = (it.seq >> 8) & 4095, sp = it.seq >> 20;
+  const int k0 = it.k0, k1 = it.k1, pos = (int)(it.pos & 0x7fffffffu);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lg = lane >> 4, t = lane & 15, gi = 4 * w + lg;
+  const size_t base = (((size_t)b * a.L + a.layer) * HKV + kvh) * a.max_seq * D + 8 * t;
+  const uint4* kp = reinterpret_cast<const uint4*>(a.k_cache + base);
+  const uint4* vp = reinterpret_cast<const uint4*>(a.v_cache + base);
+  struct Round {
+    uint4 k[BU], v[BU];
+  };
+  // group gi's keys k0 + 64 r + gi + 16 u; past the item's end its last key again (masked), so that
+  // every round issues the same loads and the waits stay exact
+  auto load = [&](Round& d, int r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < BU; ++u) {
+      const size_t o = (size_t)min(k0 + KBLK * r + gi + 16 * u, k1 - 1) * (D / 8);
+      d.k[u] = ld_stream(kp + o);
+      d.v[u] = ld_stream(vp + o);
+    }
+  };
+  // the queries' and the new row's loads first: their norms and rotations then run while the first keys
+  // are on the way
+  const float* rr = a.raw + (size_t)b * (HQ + 2 * HKV) * D + 8 * t;
+  float4 xr[8];
+  uint4 xw[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float* p = rr + (i < 2 ? 2 * kvh + i : HQ + (i - 2) * HKV + kvh) * D;  // q0, q1, k, v
+    xr[2 * i] = *reinterpret_cast<const float4*>(p);
+    xr[2 * i + 1] = *reinterpret_cast<const float4*>(p + 4);
+  }
+  xw[0] = *reinterpret_cast<const uint4*>(a.q_norm + 8 * t);
+  xw[1] = *reinterpret_cast<const uint4*>(a.k_norm + 8 * t);
+  xw[2] = *reinterpret_cast<const uint4*>(a.cos_tab + (size_t)pos * D + 8 * (t & 7));  // dims mod 64
+  xw[3] = *reinterpret_cast<const uint4*>(a.sin_tab + (size_t)pos * D + 8 * (t & 7));
+  __builtin_amdgcn_sched_barrier(0);
+  Round A, B;
+  load(A, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  float qa[8], qb[8], kn[8], vn[8], qw[8], kw[8], cs[8], sn[8];
+  auto ld8 = [&](int i, float (&v)[8]) {
+    const float4 x = xr[2 * i], y = xr[2 * i + 1];
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w; v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+  };
+  ld8(0, qa);
+  ld8(1, qb);
+  ld8(2, kn);
+  ld8(3, vn);
+  unpack8(xw[0], qw);
+  unpack8(xw[1], kw);
+  unpack8(xw[2], cs);
+  unpack8(xw[3], sn);
+  head_norm_rope(qa, qw, cs, sn, t);
+  head_norm_rope(qb, qw, cs, sn, t);
+  constexpr float QS = ATT_SCALE * 1.4426950408889634f;  // scores in base 2
+#pragma unroll
+  for (int i = 0; i < 8; ++i) { qa[i] *= QS; qb[i] *= QS; }
+  const bool ends = sp == ns - 1;  // the item that holds the new row
+  uint4 knew = make_uint4(0, 0, 0, 0), vnew = knew;
+  if (ends) {
+    head_norm_rope(kn, kw, cs, sn, t);
+    knew = make_uint4(pack_bf16x2(kn[0], kn[1]), pack_bf16x2(kn[2], kn[3]), pack_bf16x2(kn[4], kn[5]),
+                      pack_bf16x2(kn[6], kn[7]));
+    vnew = make_uint4(pack_bf16x2(vn[0], vn[1]), pack_bf16x2(vn[2], vn[3]), pack_bf16x2(vn[4], vn[5]),
+                      pack_bf16x2(vn[6], vn[7]));
+  }
+
   float m0 = -INFINITY, m1 = -INFINITY, l0 = 0.f, l1 = 0.f, a0[8], a1[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) { a0[i] = 0.f; a1[i] = 0.f; }
-  auto step = [&](float sc, const float (&v)[8], float& m, float& l, float (&acc)[8]) {
-    const float nm = fmaxf(m, sc);
-    const float cm = __expf(m - nm), e = __expf(sc - nm);
-    l = l * cm + e;
+  auto update = [&](const float (&s)[BU], const float (&vf)[BU][8], float& m, float& l, float (&acc)[8])
+      __attribute__((always_inline)) {
+    float nm = m;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = acc[i] * cm + e * v[i];
+    for (int u = 0; u < BU; ++u) nm = fmaxf(nm, s[u]);
+    const float mc = nm == -INFINITY ? 0.f : nm;  // a group without keys so far: weights 0, not NaN
+    const float cm = __builtin_amdgcn_exp2f(m - mc);
+    float e[BU];
+    l *= cm;
+#pragma unroll
+    for (int u = 0; u < BU; ++u) { e[u] = __builtin_amdgcn_exp2f(s[u] - mc); l += e[u]; }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      acc[i] *= cm;
+#pragma unroll
+      for (int u = 0; u < BU; ++u) acc[i] = fmaf(e[u], vf[u][i], acc[i]);
+    }
     m = nm;
   };
+  auto compute = [&](Round& d, int r) __attribute__((always_inline)) {
+    const int p0 = k0 + KBLK * r + gi;
+    if (ends && KBLK * (r + 1) > pos - k0) {  // the round with the new row: it and the masked keys from registers
 #pragma unroll
-  for (int u = 0; u < BU; ++u) {
-    const int p = k0 + gi + 16 * u;
-    const bool own = p == pos;  // the new row, from registers
-    float kf[8], vf[8];
-    unpack8(own ? knew : kw[u], kf);
-    unpack8(own ? vnew : vw[u], vf);
-    float d0 = 0.f, d1 = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) { d0 = fmaf(qa[i], kf[i], d0); d1 = fmaf(qb[i], kf[i], d1); }
-    d0 = row16_sum(d0) * ATT_SCALE;
-    d1 = row16_sum(d1) * ATT_SCALE;
-    if (p < k1) {
-      step(d0, vf, m0, l0, a0);
-      step(d1, vf, m1, l1, a1);
+      for (int u = 0; u < BU; ++u)
+        if (p0 + 16 * u >= pos) { d.k[u] = knew; d.v[u] = vnew; }
     }
-  }
+    float s0[BU], s1[BU], vf[BU][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) { gacc[gi][0][8 * t + i] = a0[i]; gacc[gi][1][8 * t + i] = a1[i]; }
-  if (t == 0) { gml[gi][0][0] = m0; gml[gi][0][1] = l0; gml[gi][1][0] = m1; gml[gi][1][1] = l1; }
-  __syncthreads();
-  const int h = tid >> 7, d = tid & 127;
-  float M = -INFINITY;
-  for (int q = 0; q < 16; ++q) M = fmaxf(M, gml[q][h][0]);  // finite: the split has a key
-  float A = 0.f, Ls = 0.f;
-  for (int q = 0; q < 16; ++q) {
-    const float f = __expf(gml[q][h][0] - M);  // 0 for a group without keys
-    A = fmaf(gacc[q][h][d], f, A);
-    Ls = fmaf(gml[q][h][1], f, Ls);
-  }
-  float* o = part + ((((size_t)b * HKV + kvh) * S + s) * 2 + h) * APW;
-  o[d] = A;
-  if (d == 0) { o[D] = M; o[D + 1] = Ls; }
-}
-
-// The attention of one sequence and K/V head, with the new row's projections finished here (from the
-// raw Q/K/V sums, fp32 [B][4096]): every 16-lane group normalises and rotates the pair's two query
-// heads itself, and the new K row (normalised, rotated) and V row are rounded to bf16; the workgroup
-// whose splits include the sequence's position writes them into the cache and attends to that
-// position from registers. Workgroup x takes splits x, x + gridDim.x, ... of [0, position] (the grid
-// does not depend on the device-side positions); the merge reads splits below ceil(ctx / KS) only.
-__global__ void __launch_bounds__(256) battn_partial_kernel(const float* raw, const int32_t* positions,
-                                                            const int32_t* tokens, int vocab,
-                                                            const uint16_t* q_norm, const uint16_t* k_norm,
-                                                            const uint16_t* cos_tab, const uint16_t* sin_tab,
-                                                            uint16_t* k_cache, uint16_t* v_cache, int L, int layer,
-                                                            int max_seq, float* part, int S, int32_t* bad) {
-  __shared__ float gacc[16][2][D];
-  __shared__ float gml[16][2][2];
-  const int kvh = blockIdx.y, b = blockIdx.z;
-  const int lane = threadIdx.x & 63, t = lane & 15;
-  const int pos = seq_pos(positions, b, max_seq, threadIdx.x == 0 && blockIdx.x == 0 && kvh == 0 ? bad : nullptr);
-  // a sequence whose position or token is out of range reports NaN and -1 and keeps its cache as it
-  // was: its new K/V rows are not written (the clamped position would overwrite a valid row)
-  const bool write_ok = positions[b] == pos && tokens[b] >= 0 && tokens[b] < vocab;
-  const int ctx = pos + 1;
-  if ((int)blockIdx.x * KS >= ctx) return;  // no split for this workgroup (the grid fits the longest cache)
-  // the first split's K/V rows are in flight while the new row's projections are finished
-  uint4 kw[BU], vw[BU];
-  battn_load(k_cache, v_cache, b, kvh, blockIdx.x, ctx, L, layer, max_seq, kw, vw);
-  const float* rr = raw + (size_t)b * (HQ + 2 * HKV) * D + 8 * t;
-  float qa[8], qb[8], kn[8], vv[8], qw[8], kwn[8], cs[8], sn[8];
-  auto ld8 = [](const float* p, float (&v)[8]) {
-    const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w; v[4] = y.x; v[5] = y.y; v[6] = y.z; v[7] = y.w;
+    for (int u = 0; u < BU; ++u) {
+      float kf[8];
+      unpack8(d.k[u], kf);
+      unpack8(d.v[u], vf[u]);
+      float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) { d0 = fmaf(qa[i], kf[i], d0); d1 = fmaf(qb[i], kf[i], d1); }
+      d0 = row16_sum(d0);
+      d1 = row16_sum(d1);
+      const bool in = p0 + 16 * u < k1;
+      s0[u] = in ? d0 : -INFINITY;
+      s1[u] = in ? d1 : -INFINITY;
+    }
+    update(s0, vf, m0, l0, a0);
+    update(s1, vf, m1, l1, a1);
   };
-  ld8(rr + (2 * kvh) * D, qa);
-  ld8(rr + (2 * kvh + 1) * D, qb);
-  ld8(rr + (HQ + kvh) * D, kn);
-  ld8(rr + (HQ + HKV + kvh) * D, vv);
-  unpack8(*reinterpret_cast<const uint4*>(q_norm + 8 * t), qw);
-  unpack8(*reinterpret_cast<const uint4*>(k_norm + 8 * t), kwn);
-  unpack8(*reinterpret_cast<const uint4*>(cos_tab + (size_t)pos * D + 8 * (t & 7)), cs);  // dims mod 64
-  unpack8(*reinterpret_cast<const uint4*>(sin_tab + (size_t)pos * D + 8 * (t & 7)), sn);
-  head_norm_rope(qa, qw, cs, sn, t);
-  head_norm_rope(qb, qw, cs, sn, t);
-  head_norm_rope(kn, kwn, cs, sn, t);
-  const uint4 knew = make_uint4(pack_bf16x2(kn[0], kn[1]), pack_bf16x2(kn[2], kn[3]), pack_bf16x2(kn[4], kn[5]),
-                                pack_bf16x2(kn[6], kn[7]));
-  const uint4 vnew = make_uint4(pack_bf16x2(vv[0], vv[1]), pack_bf16x2(vv[2], vv[3]), pack_bf16x2(vv[4], vv[5]),
-                                pack_bf16x2(vv[6], vv[7]));
-  if (write_ok && threadIdx.x < 16 && (pos / KS) % gridDim.x == blockIdx.x) {
-    const size_t row = ((((size_t)b * L + layer) * HKV + kvh) * max_seq + pos) * D + 8 * t;
-    *reinterpret_cast<uint4*>(k_cache + row) = knew;
-    *reinterpret_cast<uint4*>(v_cache + row) = vnew;
+  const int nr = (k1 - k0 + KBLK - 1) / KBLK;
+  for (int r = 0; r < nr; r += 2) {
+    load(B, r + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(A, r);
+    load(A, r + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    if (r + 1 < nr) compute(B, r + 1);
   }
-  for (int s = blockIdx.x; s * KS < ctx; s += gridDim.x) {
-    if (s != (int)blockIdx.x) battn_load(k_cache, v_cache, b, kvh, s, ctx, L, layer, max_seq, kw, vw);
-    battn_split(qa, qb, knew, vnew, pos, kw, vw, b, kvh, s, ctx, part, S, gacc, gml);
-    __syncthreads();  // gacc / gml are reused by the next split
+  // the new row into the cache (after the loop: a store in flight would make its waits full ones)
+  if (ends && it.pos >> 31 && tid < 16) {
+    const size_t row = base + (size_t)pos * D;
+    *reinterpret_cast<uint4*>(a.k_cache + row) = knew;
+    *reinterpret_cast<uint4*>(a.v_cache + row) = vnew;
   }
-}
 
-// Merge of the splits of each sequence and query head into the O-projection's input row (bf16 hi/lo
-// [B][2048]); 128 threads, one per dim.
-// ldo == 0: skinny fragments of the 2048 attention outputs in oh (hi and lo).
-__global__ void __launch_bounds__(128) battn_merge_kernel(const float* part, int S, const int32_t* positions,
-                                                          int max_seq, uint16_t* oh, uint16_t* ol, int ldo) {
-  const int b = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-  const int kvh = h >> 1, hh = h & 1;
-  const int pos = seq_pos(positions, b, max_seq, nullptr);
-  const float* p = part + (((size_t)b * HKV + kvh) * S * 2 + hh) * APW;
-  // The first NB splits' words are loaded together with the position (one round trip instead of one
-  // per split and pass); those past the sequence's split count are read (inside the S allocated
-  // slots) but never used.
-  constexpr int NB = 16;
-  float mv[NB], lv[NB], av[NB];
-  {
-    // lane l of each wave loads split l % NB's (m, l) pair (vector loads, issued with the rest), then
-    // every lane reads them off lanes 0..NB-1
-    const int sl = d & (NB - 1);
-    const float2 ml = *reinterpret_cast<const float2*>(p + (size_t)(sl < S ? sl : 0) * 2 * APW + D);
+  // the wave's 4 groups, then the 4 waves
+  auto merge4 = [&](float m, float l, float (&acc)[8], int h) __attribute__((always_inline)) {
+    const float mm = xmax32(xmax16(m)), mc = mm == -INFINITY ? 0.f : mm;
+    const float f = __builtin_amdgcn_exp2f(m - mc);
+    l = xsum32(xsum16(l * f));
 #pragma unroll
-    for (int s = 0; s < NB; ++s) av[s] = p[(size_t)(s < S ? s : 0) * 2 * APW + d];
-#pragma unroll
-    for (int s = 0; s < NB; ++s) {
-      mv[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.x), s));
-      lv[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ml.y), s));
+    for (int i = 0; i < 8; ++i) acc[i] = xsum32(xsum16(acc[i] * f));
+    if (lg == h) {
+      float4* o = reinterpret_cast<float4*>(&sacc[w][h][8 * t]);
+      o[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      o[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+      if (t == 0) { sml[w][h][0] = mm; sml[w][h][1] = l; }
     }
-  }
-  const int ns = (pos + KS) / KS;  // ceil((pos + 1) / KS)
-  // max first over the first NB splits, then their weighted sums in split order (selects, not
-  // branches, so that no loop separates the loads above from their use)
+  };
+  merge4(m0, l0, a0, 0);
+  merge4(m1, l1, a1, 1);
+  __syncthreads();
+  const int h = tid >> 7, d = tid & 127;  // one head and dim per thread
   float M = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < NB; ++s) M = fmaxf(M, s < ns ? mv[s] : -INFINITY);
-  float A = 0.f, Ls = 0.f;
+  for (int q = 0; q < 4; ++q) M = fmaxf(M, sml[q][h][0]);  // finite: an item has keys
+  float acc = 0.f, l = 0.f;
 #pragma unroll
-  for (int s = 0; s < NB; ++s) {
-    const bool in = s < ns;
-    const float f = in ? __expf(mv[s] - M) : 0.f;
-    A = in ? fmaf(av[s], f, A) : A;
-    Ls = in ? fmaf(lv[s], f, Ls) : Ls;
+  for (int q = 0; q < 4; ++q) {
+    const float f = __builtin_amdgcn_exp2f(sml[q][h][0] - M);  // 0 for a wave without keys
+    acc = fmaf(sacc[q][h][d], f, acc);
+    l = fmaf(sml[q][h][1], f, l);
   }
-  // splits past NB (caches longer than NB * KS keys): online, rescaling the sums to a new maximum
-  for (int s = NB; s < ns; ++s) {
-    const float* q = p + (size_t)s * 2 * APW;
-    const float m = q[D];
-    if (m > M) {
-      const float c = __expf(M - m);
-      A *= c;
-      Ls *= c;
-      M = m;
+  if (ns > 1) {
+    const __amdgpu_buffer_rsrc_t part = make_rsrc(a.part);
+    const int slot = (int)(((blockIdx.x >> 3) * HKV + kvh) * 2 + h) * APW;  // floats
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc), part, 4 * (slot + d), 0, CPOL_SC1);
+    if (d < 2) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(d ? l : M), part, 4 * (slot + D + d), 0, CPOL_SC1);
+    wait_vmem();  // acknowledged before this workgroup counts itself
+    __syncthreads();
+    if (tid == 0)
+      arrived = __hip_atomic_fetch_add(a.count + b * HKV + kvh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if ((int)arrived != ns - 1) return;
+    if (tid == 0) st_dev_u32(a.count + b * HKV + kvh, 0);  // for the next layer
+    constexpr int NB = 8;  // splits whose words are loaded together
+    const int s00 = (int)((((blockIdx.x >> 3) - sp) * HKV + kvh) * 2 + h) * APW, stride = HKV * 2 * APW;
+    M = -INFINITY;
+    acc = 0.f;
+    l = 0.f;
+    for (int s = 0; s < ns; s += NB) {
+      float av[NB], mv[NB], lv[NB];
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const int o = s00 + min(s + q, ns - 1) * stride;
+        av[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(part, 4 * (o + d), 0, CPOL_SC1));
+        mv[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(part, 4 * (o + D), 0, CPOL_SC1));
+        lv[q] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(part, 4 * (o + D + 1), 0, CPOL_SC1));
+      }
+      float nm = M;
+#pragma unroll
+      for (int q = 0; q < NB; ++q) nm = fmaxf(nm, mv[q]);
+      const float c = __builtin_amdgcn_exp2f(M - nm);
+      acc *= c;
+      l *= c;
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const float f = s + q < ns ? __builtin_amdgcn_exp2f(mv[q] - nm) : 0.f;
+        acc = fmaf(av[q], f, acc);
+        l = fmaf(lv[q], f, l);
+      }
+      M = nm;
     }
-    const float f = __expf(m - M);
-    A = fmaf(q[d], f, A);
-    Ls = fmaf(q[D + 1], f, Ls);
   }
-  const float o = A / Ls;
-  const uint16_t hi = f32_to_bf16(o), lo = f32_to_bf16(o - bf16_to_f32(hi));
-  if (ldo == 0) {
-    oh[skf_off(b, h * D + d, 0, gridDim.x, HQ * D)] = hi;
-    oh[skf_off(b, h * D + d, 1, gridDim.x, HQ * D)] = lo;
-  } else {
-    oh[(size_t)b * ldo + h * D + d] = hi;
-    ol[(size_t)b * ldo + h * D + d] = lo;
+  so[h][d] = acc / l;
+  __syncthreads();
+  if (tid < 2 * D / 8) {  // 8 dims of one head per thread
+    const int hh = tid >> 4, c = 8 * (tid & 15);
+    float o[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = so[hh][c + i];
+    uint4 hi, lo;
+    split8(o, hi, lo);
+    const int k = (2 * kvh + hh) * D + c;
+    *reinterpret_cast<uint4*>(a.out + skf_off(b, k, 0, a.B, HQ * D)) = hi;
+    *reinterpret_cast<uint4*>(a.out + skf_off(b, k, 1, a.B, HQ * D)) = lo;
   }
 }
 
@@ -1875,26 +1975,31 @@ namespace mkp {
 
 // Split-K factors of the O and down products (each wave's K range a multiple of 256)
 
+// Workspace: what grows with the batch in either engine first (residual rows, keys, counters, plan),
+// then, from `rest` on, this engine's other areas -- or the persistent engine's, which share the space.
 struct BLayout {
-  size_t x, ah, al, af, bf, raw, part, apart, keys, bad, bytes;
+  size_t x, keys, bad, count, plan, rest, ah, al, af, bf, raw, part, apart, bytes;
 };
-static BLayout blayout(int H, int I, int B, int max_seq) {
+static BLayout blayout(int H, int I, int B) {
   const size_t A = H > HQ * D ? H : HQ * D;
-  const int S = (max_seq + KS - 1) / KS;
   BLayout L;
   size_t o = 0;
   auto take = [&](size_t n) { const size_t r = o; o += align256(n); return r; };
   L.x = take((size_t)B * H * 4);
+  L.keys = take((size_t)B * 8);
+  L.bad = take(4);
+  L.count = take((size_t)B * HKV * 4);
+  L.plan = take((size_t)plan_items(B) * sizeof(PlanItem));
+  L.rest = o;
   L.ah = take(frag_rows(B) * A * 2);  // whole row tiles for the LM head's gemm_kernel
   L.al = take(frag_rows(B) * A * 2);
   L.af = take(skf_elems(B, (int)A) * 2);  // skinny fragments: the QKV, O and gate/up inputs
   L.bf = take(skf_elems(B, I) * 2);       // ... and the down input
   L.raw = take((size_t)B * (HQ + 2 * HKV) * D * 4);
   L.part = take((size_t)3 * B * H * 4);
-  L.apart = take((size_t)B * HKV * S * 2 * APW * 4);
-  L.keys = take((size_t)B * 8);
-  L.bad = take(4);
+  L.apart = take((size_t)plan_items(B) * HKV * 2 * APW * 4);
   L.bytes = o;
+  if (B <= 2 * MKB_MAX && L.bytes < L.rest + mkb_workspace_bytes()) L.bytes = L.rest + align256(mkb_workspace_bytes());
   return L;
 }
 
@@ -1906,7 +2011,6 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
                             char* ws, const BLayout& Lo, hipStream_t st) {
   typedef BatchPlan<H, I> BP;
   const int A = H > HQ * D ? H : HQ * D;
-  const int S = (max_seq + KS - 1) / KS;
   float* x = reinterpret_cast<float*>(ws + Lo.x);
   uint16_t* ah = reinterpret_cast<uint16_t*>(ws + Lo.ah);
   uint16_t* al = reinterpret_cast<uint16_t*>(ws + Lo.al);
@@ -1917,6 +2021,8 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
   float* apart = reinterpret_cast<float*>(ws + Lo.apart);
   u64* keys = reinterpret_cast<u64*>(ws + Lo.keys);
   int32_t* bad = reinterpret_cast<int32_t*>(ws + Lo.bad);
+  uint32_t* count = reinterpret_cast<uint32_t*>(ws + Lo.count);
+  PlanItem* plan = reinterpret_cast<PlanItem*>(ws + Lo.plan);
   const int L = dims.num_layers;
   hipError_t e;
 #define MKB_LAUNCH(...)                                   \
@@ -1924,11 +2030,9 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
     hipLaunchKernelGGL(__VA_ARGS__);                      \
     if ((e = hipGetLastError()) != hipSuccess) return e;  \
   } while (0)
-  MKB_LAUNCH(keys_init_kernel, dim3(1), dim3(64), 0, st, keys, B, bad);
+  MKB_LAUNCH(batch_plan_kernel, dim3(1), dim3(64), 0, st, positions, tokens, dims.vocab, max_seq, B, keys, bad, count,
+             plan);
   const int cb = column_blocks(B);
-  // attention workgroups per sequence and K/V head (each loops over its splits): about 1024 in all,
-  // 16 at most (the grid cannot follow the device-side positions, so it must not be mostly idle)
-  const int gx = B <= 8 ? 16 : B <= 16 ? 8 : B <= 32 ? 4 : 2;
   const dim3 rows(B), nthr(64);  // norms: one row per single-wave workgroup
   const int so = BP::SO, sd = BP::SD;
   for (int l = 0; l < L; ++l) {
@@ -1941,10 +2045,9 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
     q.w0 = (const uint16_t*)lw.q_weight; q.w1 = (const uint16_t*)lw.k_weight; q.w2 = (const uint16_t*)lw.v_weight;
     q.n1 = HQ * D; q.n2 = (HQ + HKV) * D; q.out = raw;
     if ((e = launch_skinny(SK_RAW, cb, dim3(q.N / 16, 1), q, st)) != hipSuccess) return e;
-    MKB_LAUNCH(battn_partial_kernel, dim3(S < gx ? S : gx, HKV, B), dim3(256), 0, st, raw, positions, tokens,
-               dims.vocab, (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab, k_cache,
-               v_cache, L, l, max_seq, apart, S, bad);
-    MKB_LAUNCH(battn_merge_kernel, dim3(B, HQ), dim3(D), 0, st, apart, S, positions, max_seq, af, nullptr, 0);
+    const BAttnArgs at{raw, (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab,
+                       k_cache, v_cache, L, l, max_seq, B, plan, apart, count, af};
+    MKB_LAUNCH(battn_kernel, dim3(plan_items(B) * HKV), dim3(256), 0, st, at);
     SkArgs o{};
     o.xh = af; o.B = B; o.N = H; o.K = HQ * D; o.w0 = (const uint16_t*)lw.o_proj_weight; o.out = part;
     if ((e = launch_skinny(SK_PART, cb, dim3(H / 16, so), o, st)) != hipSuccess) return e;
@@ -1993,9 +2096,7 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
 // The larger of the two engines' needs, so that the engine can be chosen per call.
 extern "C" size_t mk_decode_batch_workspace_bytes(const mk_model_dims* dims, int batch, int max_seq_len) {
   if (!dims || batch < 1 || batch > BMAX || max_seq_len < 1) return 0;
-  const size_t n = blayout(dims->hidden, dims->intermediate, batch, max_seq_len).bytes;
-  const size_t p = mkb_workspace_bytes();
-  return batch <= 2 * MKB_MAX && p > n ? p : n;
+  return blayout(dims->hidden, dims->intermediate, batch).bytes;
 }
 
 extern "C" hipError_t mk_decode_batch(const mk_model_dims* dims, int batch, const int32_t* tokens,
@@ -2012,13 +2113,13 @@ extern "C" hipError_t mk_decode_batch(const mk_model_dims* dims, int batch, cons
   if (!(s06 || s17) || dims->num_layers < 1 || dims->vocab < 1) return hipErrorInvalidValue;
   if (batch < 1 || batch > BMAX || max_seq_len < 1) return hipErrorInvalidValue;
   if (dims->vocab % 16 != 0) return hipErrorInvalidValue;  // the LM head's skinny product takes 16 rows per workgroup
-  const BLayout Lo = blayout(dims->hidden, dims->intermediate, batch, max_seq_len);
+  const BLayout Lo = blayout(dims->hidden, dims->intermediate, batch);
   if (workspace_bytes < Lo.bytes || reinterpret_cast<uintptr_t>(workspace) % 256 != 0) return hipErrorInvalidValue;
   const mk_layer_weights* lw = static_cast<const mk_layer_weights*>(layer_weights);  // host array
+  char* ws = static_cast<char*>(workspace);
   if (mkb_applies(dims, batch, max_seq_len)) {
-    if (workspace_bytes < mkb_workspace_bytes()) return hipErrorInvalidValue;
     return mkb_decode_batch(dims, batch, tokens, positions, embed_weight, lm_head_weight, final_norm_weight, lw,
-                            cos_table, sin_table, k_cache, v_cache, max_seq_len, logits, out_tokens, workspace,
+                            cos_table, sin_table, k_cache, v_cache, max_seq_len, logits, out_tokens, ws + Lo.rest,
                             stream);
   }
   // 17-24 sequences (17-32 with the persistent engine forced) where the persistent kernel applies
@@ -2030,19 +2131,18 @@ extern "C" hipError_t mk_decode_batch(const mk_model_dims* dims, int batch, cons
   const int two_max = mkb_engine() == 2 ? 2 * MKB_MAX : MKB_MAX + 8;
   if (batch > MKB_MAX && batch <= two_max && mkb_applies(dims, MKB_MAX, max_seq_len) &&
       mkb_applies(dims, batch - MKB_MAX, max_seq_len)) {
-    if (workspace_bytes < mkb_workspace_bytes()) return hipErrorInvalidValue;
     const size_t seq_cache = (size_t)dims->num_layers * HKV * max_seq_len * D;  // elements per sequence
     for (int b0 = 0; b0 < batch; b0 += MKB_MAX) {
       const int nb = batch - b0 < MKB_MAX ? batch - b0 : MKB_MAX;
       const hipError_t e = mkb_decode_batch(
           dims, nb, tokens + b0, positions + b0, embed_weight, lm_head_weight, final_norm_weight, lw, cos_table,
           sin_table, static_cast<uint16_t*>(k_cache) + b0 * seq_cache, static_cast<uint16_t*>(v_cache) + b0 * seq_cache,
-          max_seq_len, logits + (size_t)b0 * dims->vocab, out_tokens ? out_tokens + b0 : nullptr, workspace, stream);
+          max_seq_len, logits + (size_t)b0 * dims->vocab, out_tokens ? out_tokens + b0 : nullptr, ws + Lo.rest,
+          stream);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
   }
-  char* ws = static_cast<char*>(workspace);
   if (s06)
     return run_batch<1024, 3072>(*dims, batch, tokens, positions, (const uint16_t*)embed_weight,
                                  (const uint16_t*)lm_head_weight, (const uint16_t*)final_norm_weight, lw,

@@ -74,6 +74,10 @@ def engine(request):
     ("mini", (7, 300, 45, 128, 256, 99, 1, 410, 64), 3, 2),  # 9 sequences: a second column block of one
     ("mini", tuple(2 + 31 * i for i in range(16)), 3, 2),  # 16 sequences: two full column blocks
     ("mini2k", (1900, 50, 1000, 1500, 300, 2000, 17, 800, 1200, 640, 1, 1750), 2, 2),  # 12 long: 32 ranges of 448
+    # layer by layer, key ranges per sequence: 32 of one block each; up to 5 blocks each in one or several
+    ("mini2k", (2000,), 2, 1),
+    ("mini2k", tuple(1 + 97 * i for i in range(20)), 2, 1),
+    ("mini2k", (62, 63, 64, 1279, 1280, 1407), 2, 1),     # positions at the edges of key blocks
     ("mini17", (33, 200, 90), 4, 1),
     ("mini17", tuple(5 + 37 * i for i in range(12)), 2, 1),  # 1.7B width, 12 sequences: register-blocked products
     ("mini", tuple(3 + 11 * i for i in range(20)), 2, 1),  # 20 sequences: 3 column blocks of 8 (of 4)
