@@ -23,8 +23,8 @@
 // are split over K too, into raw sums that qkv_post_kernel / silu_post_kernel finish. The attention
 // takes one query block per workgroup, or key-range chunks of the blocks merged by
 // attn_merge_kernel where the blocks' key chains are uneven against the grid. Prompts of at most
-// small_m(H) tokens run the products on the skinny kernels of the batched decode instead (weights
-// as the MFMA A operand, activations in its skinny fragment order).
+// SMALL_M tokens run the products on the skinny kernels of the batched decode instead (weights
+// as the MFMA A operand, activations in its skinny fragment order, the norms folded into the products).
 //
 // Numerics are the decode kernel's (the reference kernel's fp32 design, /root/reference/
 // megakernel.cu): fp32 residual and accumulation, fp32 RMSNorm, exact softmax, new K/V rounded to
@@ -1008,120 +1008,260 @@ __global__ void keys_to_tokens_kernel(const u64* keys, int R, const int32_t* bad
 // ------------------------------------------------------------------------------------------------
 constexpr int BMAX = 64;
 
-enum SkEpi { SK_RAW = 0, SK_PART = 1, SK_SILU = 2 };
+enum SkEpi { SK_RAW = 0, SK_RESID = 1, SK_SILU = 2 };
 
+// The RMSNorms between the skinny products have no kernel of their own. A norm is
+// x[b][k] * w[k] * rs[b] with rs[b] = rsqrt(mean_k x[b][k]^2 + eps), and a product is linear in its
+// input rows, so the product that completes the residual x (SK_RESID) writes x * w as the next
+// product's fragments and, per 16-row tile, each row's sum of squares; the product that reads them
+// (SK_RAW, SK_SILU) scales its sums by rs[b]. (The decode kernel splits its norms the same way.)
 struct SkArgs {
   const uint16_t* xh;  // activations as skinny fragments (skf_off: K inputs, hi and lo) of B rows
   int B, N, K;
-  // SK_RAW: rows [0, n1) of w0, [n1, n2) of w1, [n2, N) of w2 (Q, K, V); SK_PART: w0; SK_SILU: w0 gate, w1 up
+  // SK_RAW: rows [0, n1) of w0, [n1, n2) of w1, [n2, N) of w2 (Q, K, V); SK_RESID: w0; SK_SILU: w0 gate, w1 up
   const uint16_t* w0;
   const uint16_t* w1;
   const uint16_t* w2;
   int n1, n2;
-  float* out;    // SK_RAW: [B][N]; SK_PART: [gridDim.y][B][N]
-  uint16_t* mh;  // SK_SILU: silu(gate) * up as skinny fragments of ldm inputs (the down product's operand)
+  const float* ssq;  // SK_RAW, SK_SILU: [K / 16][B] sums of squares of the input rows; null: no scale
+  float* out;        // SK_RAW: [B][N]; SK_RESID: the residual x [B][N], updated in place
+  // SK_SILU: silu(gate) * up, SK_RESID (null: not wanted): the new x * norm, as skinny fragments of ldm inputs
+  uint16_t* mh;
   int ldm;
+  const uint16_t* norm;  // SK_RESID: the next norm's weights [N]
+  float* ssq_out;        // SK_RESID: [N / 16][B]
 };
 
-
-// A workgroup takes 16 weight rows (rows 16 bx ..). SK_RAW / SK_PART: its K range [by K / gy, ...)
-// split over the 4 waves; SK_SILU: 8 intermediates, their 8 gate rows and 8 up rows in one 16-row
-// tile, K split over the 4 waves. Each wave's K range is a multiple of 256 (checked on the host).
-// The B operand holds CB column blocks of 8 rows of activations (a decode batch, or up to 64 prompt
+// A workgroup of W waves takes RT tiles of 16 weight rows (SK_SILU: the 8 gate and 8 up rows of 8
+// intermediates in each) and CB of the column blocks (blocks CB by ..), K split over the waves, each
+// wave's range a multiple of 32 U (checked on the host).
+// The B operand holds column blocks of 8 rows of activations (a decode batch, or up to 64 prompt
 // tokens): column li of block cb is row 8 cb + li / 2, hi (even li) or lo (odd li), read as skinny
-// fragments (skf_off) of the CB column blocks. The weight fragments of a K chunk stay in registers
-// across the column blocks; up to 4 blocks' activation fragments are in flight while a block is
-// multiplied.
-template <int EPI, int CB>
-__global__ void __launch_bounds__(256) skinny_kernel(const SkArgs g) {
-  constexpr int NC = 8 * CB;
-  __shared__ float red[4][16][NC + 1];
+// fragments (skf_off). The weight fragments of a K chunk stay in registers across the column blocks, a
+// block's activation fragments across the row tiles; the loads of up to 4 blocks are in flight at once.
+//
+// Weight loads: an MFMA operand holds 64 bytes of each of 16 rows, but a load instruction that takes
+// 64 bytes of 16 rows streams worse than one that takes 128 bytes (a cache line) of 8. So a pair of
+// loads takes 64 inputs of rows 0-7 and of rows 8-15, lane li reading chunk 4 (li / 8) + lg of row
+// li % 8, and the halves trade places in registers (row_ror:8 inside 16 lanes).
+template <int EPI, int W, int U, int RT, int CB>
+__global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
+  constexpr int NC = 8 * CB, NT = 64 * W, ROWS = 16 * RT;
+  static_assert(U % 2 == 0, "weight loads come in pairs");
+  __shared__ float red[W][ROWS][NC + 1];
+  __shared__ float rsp[NT];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  const int n0 = 16 * blockIdx.x, n = n0 + li;
-  const uint16_t* wrow;
-  int kb, ke;
-  if constexpr (EPI == SK_SILU) {
-    wrow = (li < 8 ? g.w0 : g.w1) + (size_t)(8 * blockIdx.x + (li & 7)) * g.K;
-    const int kw = g.K / 4;
-    kb = w * kw;
-    ke = kb + kw;
-  } else {
-    if constexpr (EPI == SK_RAW)
-      wrow = n < g.n1 ? g.w0 + (size_t)n * g.K
-                      : (n < g.n2 ? g.w1 + (size_t)(n - g.n1) * g.K : g.w2 + (size_t)(n - g.n2) * g.K);
-    else
-      wrow = g.w0 + (size_t)n * g.K;
-    const int kc = g.K / gridDim.y, kw = kc / 4;
-    kb = blockIdx.y * kc + w * kw;
-    ke = kb + kw;
-  }
-  const int sb = li >> 1;
-  f32x4 c[CB];
+  const int c0 = CB * blockIdx.y, b0 = 8 * c0;  // first column block and activation row
+  const int CBT = CB * gridDim.y;               // column blocks of the fragments
+  const int nb = min(g.B - b0, NC);             // activation rows of this workgroup
+  // this lane's weight rows: tile rt, rows li % 8 and 8 + li % 8
+  const uint16_t* wp[RT][2];
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb) c[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const int tile = RT * blockIdx.x + rt, n = 16 * tile + 8 * hf + (li & 7);
+      const uint16_t* row;
+      if constexpr (EPI == SK_SILU)
+        row = (hf ? g.w1 : g.w0) + (size_t)(8 * tile + (li & 7)) * g.K;
+      else if constexpr (EPI == SK_RAW)
+        row = n < g.n1 ? g.w0 + (size_t)n * g.K
+                       : (n < g.n2 ? g.w1 + (size_t)(n - g.n1) * g.K : g.w2 + (size_t)(n - g.n2) * g.K);
+      else
+        row = g.w0 + (size_t)n * g.K;
+      wp[rt][hf] = row + 8 * (4 * (li >> 3) + lg);
+    }
+  // the rows' sums of squares: NT / NC threads per row, each a share of the K / 16 tiles
+  constexpr int P = NT / NC;
+  constexpr int MAXT = (2048 / 16 + P - 1) / P;  // tiles per thread at the widest input
+  float sq[MAXT];
+  if constexpr (EPI != SK_RESID) {
+    if (g.ssq) {
+      const int b = min(b0 + tid % NC, g.B - 1), t0 = tid / NC;
+#pragma unroll
+      for (int i = 0; i < MAXT; ++i) sq[i] = g.ssq[(size_t)min(t0 + P * i, g.K / 16 - 1) * g.B + b];
+    }
+  }
+  // SK_RESID: this thread's residual values (idx = tid + NT i: row idx % ROWS of activation row idx / ROWS)
+  constexpr int EPT = (ROWS * NC + NT - 1) / NT;
+  float xo[EPT], nw[EPT];
+  if constexpr (EPI == SK_RESID) {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const int idx = tid + NT * i, b = min(b0 + idx / ROWS, g.B - 1), n = ROWS * blockIdx.x + idx % ROWS;
+      xo[i] = g.out[(size_t)b * g.N + n];
+      nw[i] = g.mh ? bf16_to_f32(g.norm[n]) : 0.f;
+    }
+  }
+  const int kw = g.K / W, kb = w * kw, ke = kb + kw;
+  f32x4 c[RT][CB];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) c[rt][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4* xf = reinterpret_cast<const uint4*>(g.xh) + lane;  // this lane's 16 bytes of fragment 0
-  auto ld_act = [&](int cb, int k) { return xf[skf_frag(cb, k >> 5, CB, g.K) * 64]; };
+  auto ld_act = [&](int cb, int k) { return xf[skf_frag(c0 + cb, k >> 5, CBT, g.K) * 64]; };
   // R column blocks' activation fragments in flight: block cb + R's loads go into the registers
   // block cb's MFMAs have just read (no copies: a register copy of a pending load would wait for it)
   constexpr int R = CB < 4 ? CB : 4;
-  for (int k0 = kb; k0 < ke; k0 += 256) {
-    uint4 wa[8], xq[R][8];
+  for (int k0 = kb; k0 < ke; k0 += 32 * U) {
+    uint4 wa[RT][U], xq[R][U];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) wa[u] = ld_stream(reinterpret_cast<const uint4*>(wrow + k0 + 32 * u + 8 * lg));
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        wa[rt][u] = ld_stream(reinterpret_cast<const uint4*>(wp[rt][u & 1] + k0 + 64 * (u >> 1)));
 #pragma unroll
     for (int r = 0; r < R; ++r) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) xq[r][u] = ld_act(r, k0 + 32 * u);
+      for (int u = 0; u < U; ++u) xq[r][u] = ld_act(r, k0 + 32 * u);
       __builtin_amdgcn_sched_barrier(0);  // the blocks' loads in block order: each wait covers one block
     }
+    // operand u: rows 0-7 from the first load's lower lanes, rows 8-15 from the second's; operand u + 1:
+    // their upper lanes
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int u = 0; u < U; u += 2) {
+        const uint4 p = wa[rt][u], q = wa[rt][u + 1];
+        auto up = [](uint32_t a, uint32_t b) { return (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false); };
+        auto dn = [](uint32_t a, uint32_t b) { return (uint32_t)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0x3, false); };
+        wa[rt][u] = make_uint4(up(p.x, q.x), up(p.y, q.y), up(p.z, q.z), up(p.w, q.w));
+        wa[rt][u + 1] = make_uint4(dn(q.x, p.x), dn(q.y, p.y), dn(q.z, p.z), dn(q.w, p.w));
+      }
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) c[cb] = mfma(wa[u], xq[cb % R][u], c[cb]);
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) c[rt][cb] = mfma(wa[rt][u], xq[cb % R][u], c[rt][cb]);
       if (cb + R < CB) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) xq[cb % R][u] = ld_act(cb + R, k0 + 32 * u);
+        for (int u = 0; u < U; ++u) xq[cb % R][u] = ld_act(cb + R, k0 + 32 * u);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   // C[row 4 lg + j][column li]: activation row 8 cb + li / 2 is the sum of its hi and lo columns
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float v = c[cb][j] + __shfl_xor(c[cb][j], 1);
-      if (!(li & 1)) red[w][4 * lg + j][8 * cb + sb] = v;
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float v = c[rt][cb][j] + dpp<0xB1>(c[rt][cb][j]);
+        if (!(li & 1)) red[w][16 * rt + 4 * lg + j][8 * cb + (li >> 1)] = v;
+      }
+  if constexpr (EPI != SK_RESID) {
+    float t = 0.f;
+    if (g.ssq) {
+#pragma unroll
+      for (int i = 0; i < MAXT; ++i) t += tid / NC + P * i < g.K / 16 ? sq[i] : 0.f;
     }
+    rsp[tid] = t;
+  }
   __syncthreads();
-  for (int idx = tid; idx < (EPI == SK_SILU ? 8 : 16) * g.B; idx += 256) {
-    const int r = idx / g.B, b = idx % g.B;
-    if constexpr (EPI == SK_SILU) {
-      const float gt = ((red[0][r][b] + red[1][r][b]) + red[2][r][b]) + red[3][r][b];
-      const float up = ((red[0][r + 8][b] + red[1][r + 8][b]) + red[2][r + 8][b]) + red[3][r + 8][b];
-      const float m = gt / (1.f + expf(-gt)) * up;
+  auto sum = [&](int r, int b) {  // row r, column b of the tile over the waves' K ranges, in order
+    float v = red[0][r][b];
+#pragma unroll
+    for (int q = 1; q < W; ++q) v += red[q][r][b];
+    return v;
+  };
+  auto scale = [&](int b) {
+    if (!g.ssq) return 1.f;
+    float t = rsp[b];
+#pragma unroll
+    for (int q = 1; q < P; ++q) t += rsp[q * NC + b];
+    return rsqrtf(t / (float)g.K + EPS);
+  };
+  if constexpr (EPI == SK_SILU) {
+    for (int idx = tid; idx < 8 * RT * nb; idx += NT) {
+      const int i = idx % (8 * RT), b = idx / (8 * RT), r = 16 * (i >> 3) + (i & 7);
+      const float rs = scale(b), gt = sum(r, b) * rs, up = sum(r + 8, b) * rs;
+      const float m = gt / (1.f + expf(-gt)) * up;  // silu(gate) * up (/root/reference/megakernel.cu:659-665)
       const uint16_t hi = f32_to_bf16(m), lo = f32_to_bf16(m - bf16_to_f32(hi));
-      const int it = 8 * blockIdx.x + r;  // into the down product's skinny fragments (g.ldm inputs)
-      g.mh[skf_off(b, it, 0, g.B, g.ldm)] = hi;
-      g.mh[skf_off(b, it, 1, g.B, g.ldm)] = lo;
-    } else {
-      const float v = ((red[0][r][b] + red[1][r][b]) + red[2][r][b]) + red[3][r][b];
-      g.out[((size_t)blockIdx.y * g.B + b) * g.N + n0 + r] = v;
+      const int it = 8 * RT * blockIdx.x + i;  // into the down product's skinny fragments (g.ldm inputs)
+      g.mh[skf_off(b0 + b, it, 0, g.B, g.ldm)] = hi;
+      g.mh[skf_off(b0 + b, it, 1, g.B, g.ldm)] = lo;
+    }
+  } else if constexpr (EPI == SK_RAW) {
+    for (int idx = tid; idx < ROWS * nb; idx += NT) {
+      const int r = idx % ROWS, b = idx / ROWS;
+      g.out[(size_t)(b0 + b) * g.N + ROWS * blockIdx.x + r] = sum(r, b) * scale(b);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {  // the 16 rows of a tile and one b: a 16-lane row
+      const int idx = tid + NT * i, r = idx % ROWS, b = idx / ROWS, n = ROWS * blockIdx.x + r;
+      if (b < nb) {
+        const float v = xo[i] + sum(r, b);
+        g.out[(size_t)(b0 + b) * g.N + n] = v;
+        if (g.mh) {
+          const float y = v * nw[i];
+          const uint16_t hi = f32_to_bf16(y), lo = f32_to_bf16(y - bf16_to_f32(hi));
+          g.mh[skf_off(b0 + b, n, 0, g.B, g.ldm)] = hi;
+          g.mh[skf_off(b0 + b, n, 1, g.B, g.ldm)] = lo;
+          const float q = row16_sum(v * v);
+          if ((r & 15) == 0) g.ssq_out[(size_t)(n >> 4) * g.B + b0 + b] = q;
+        }
+      }
     }
   }
 }
 
-
-// The skinny product for up to 8 * cb activation rows (cb: 1, 2, 4 or 8 column blocks).
-static hipError_t launch_skinny(int epi, int cb, dim3 grid, const SkArgs& a, hipStream_t st) {
-#define MK_SK(E, C) hipLaunchKernelGGL((skinny_kernel<E, C>), grid, dim3(256), 0, st, a)
-#define MK_SK_CB(E) \
-  if (cb == 1) MK_SK(E, 1); else if (cb == 2) MK_SK(E, 2); else if (cb == 4) MK_SK(E, 4); else MK_SK(E, 8)
-  if (epi == SK_RAW) { MK_SK_CB(SK_RAW); } else if (epi == SK_PART) { MK_SK_CB(SK_PART); } else { MK_SK_CB(SK_SILU); }
-#undef MK_SK_CB
-#undef MK_SK
+template <int EPI, int W, int U, int RT, int CB>
+static hipError_t run_skinny(int cbt, const SkArgs& a, hipStream_t st) {
+  const int tiles = a.N / (EPI == SK_SILU ? 8 : 16);
+  if (a.K % (32 * W * U) != 0 || cbt % CB != 0 || tiles % RT != 0) return hipErrorInvalidValue;  // cannot happen
+  hipLaunchKernelGGL((skinny_kernel<EPI, W, U, RT, CB>), dim3(tiles / RT, cbt / CB), dim3(64 * W), 0, st, a);
   return hipGetLastError();
+}
+
+// The skinny product for up to 8 * cbt activation rows (cbt: 1, 2, 4 or 8 column blocks).
+// Every CU reads its workgroups' weight rows and all the activations of their column blocks through its
+// L1 (64 bytes per clock): at 64 rows the activations are 8 times a 16-row tile's weights. So a launch
+// takes about 256 workgroups, one per CU, and where 16-row tiles alone would give more, or one column
+// block the most traffic, a workgroup takes several tiles (RT) and a part of the column blocks (CB): per
+// CU at 64 rows (0.6B) QKV 288 -> 192 KB, gate/up 576 (the CUs with two workgroups) -> 224 KB. Measured
+// in isolation on MI355X with fresh weights, us per launch at 8 / 16 / 32 / 64 rows, against one tile
+// and all column blocks per workgroup of 4 waves, 64-byte weight segments and (O, down) the residual
+// read in the epilogue:
+//   0.6B QKV 4.6 / 5.1 / 6.5 / 8.6 -> 4.4 / 4.8 / 5.6 / 7.2, O 6.0 / 6.0 / 6.0 / 6.8 -> 5.3 / 5.2 / 5.3 /
+//   6.0, gate/up 6.5 / 7.3 / 9.4 / 12.9 -> 6.0 / 6.0 / 7.3 / 9.0, down 7.9 / 7.8 / 7.6 / 8.7 -> 6.8 /
+//   6.6 / 6.6 / 7.9;
+//   1.7B at 8 / 16 rows QKV 8.0 / 8.5 -> 6.4 / 7.0, O 6.4 / 6.5 -> 5.5 / 5.6, gate/up 15.9 / 16.4 ->
+//   12.5 / 13.2, down 13.6 / 13.3 -> 11.2 / 11.0
+// (an empty launch takes 2.5 us, one that only reads 8 / 24 / 48 MB 2.9 / 5.6 / 9.6 us). Other wave
+// counts and chunk sizes (W 4, 8, 12, 16 x U 2 .. 16) were within 3% of these or slower.
+template <int EPI>
+static hipError_t launch_skinny(int cbt, const SkArgs& a, hipStream_t st) {
+  if constexpr (EPI == SK_RAW) {
+    if (cbt == 8 && (a.N / 16) % 2 == 0) return run_skinny<EPI, 8, 4, 2, 4>(cbt, a, st);
+    if (a.K <= 1024) {
+      if (cbt == 1) return run_skinny<EPI, 8, 4, 1, 1>(cbt, a, st);
+      if (cbt == 2) return run_skinny<EPI, 8, 4, 1, 2>(cbt, a, st);
+      return run_skinny<EPI, 8, 4, 1, 4>(cbt, a, st);
+    }
+    if (cbt == 1) return run_skinny<EPI, 4, 8, 1, 1>(cbt, a, st);
+    if (cbt == 2) return run_skinny<EPI, 4, 8, 1, 2>(cbt, a, st);
+    return run_skinny<EPI, 4, 8, 1, 4>(cbt, a, st);
+  } else if constexpr (EPI == SK_RESID) {
+    const int wgs = a.N / 16 * cbt;  // with one column block each
+    if (wgs <= 256) return run_skinny<EPI, 8, 4, 1, 1>(cbt, a, st);
+    if (wgs <= 512) return a.K > 3072 ? run_skinny<EPI, 8, 8, 1, 2>(cbt, a, st) : run_skinny<EPI, 4, 8, 1, 2>(cbt, a, st);
+    return a.K > 3072 ? run_skinny<EPI, 8, 8, 1, 4>(cbt, a, st) : run_skinny<EPI, 4, 8, 1, 4>(cbt, a, st);
+  } else {
+    if (cbt == 1) return run_skinny<EPI, 4, 8, 1, 1>(cbt, a, st);
+    if (a.K <= 1024) {
+      if (cbt == 2) return run_skinny<EPI, 4, 8, 2, 2>(cbt, a, st);
+      if (cbt == 4) return run_skinny<EPI, 8, 4, 3, 2>(cbt, a, st);
+      return run_skinny<EPI, 8, 4, 3, 4>(cbt, a, st);
+    }
+    if (cbt == 2) return run_skinny<EPI, 4, 8, 3, 2>(cbt, a, st);
+    if (cbt == 4) return run_skinny<EPI, 4, 8, 3, 4>(cbt, a, st);
+    return run_skinny<EPI, 4, 4, 3, 8>(cbt, a, st);
+  }
 }
 static int column_blocks(int rows) { return rows <= 8 ? 1 : rows <= 16 ? 2 : rows <= 32 ? 4 : 8; }
 
@@ -1625,14 +1765,26 @@ __global__ void __launch_bounds__(256) battn_kernel(const BAttnArgs a) {
 // ------------------------------------------------------------------------------------------------
 // Host side
 // ------------------------------------------------------------------------------------------------
+// The half of a layer after the attention, on the skinny kernels, for B rows: O into the residual, gate/up
+// with SiLU, down into the residual. af: the attention's output; yf, ssq: the residual's norm products,
+// read and written; next: the next layer's input norm (null: the last layer); bf: the down input.
 template <int H, int I>
-struct BatchPlan {  // K splits of the skinny O and down products
-  static constexpr int SO = H == 1024 ? 2 : 2;  // O: K = 2048
-  static constexpr int SD = H == 1024 ? 3 : 2;  // down: K = I
-  static constexpr int SP = SO > SD ? SO : SD;
-  static_assert((HQ * D / SO / 4) % 256 == 0 && (I / SD / 4) % 256 == 0 && (H / 4) % 256 == 0 && (H / 2) % 256 == 0,
-                "wave K ranges must be multiples of 256");
-};
+static hipError_t skinny_mlp(const mk_layer_weights& lw, const uint16_t* next, int cb, int B, const uint16_t* af,
+                             uint16_t* yf, uint16_t* bf, float* x, float* ssq, hipStream_t st) {
+  hipError_t e;
+  SkArgs o{};
+  o.xh = af; o.B = B; o.N = H; o.K = HQ * D; o.w0 = (const uint16_t*)lw.o_proj_weight; o.out = x;
+  o.norm = (const uint16_t*)lw.post_attn_norm_weight; o.mh = yf; o.ldm = H; o.ssq_out = ssq;
+  if ((e = launch_skinny<SK_RESID>(cb, o, st)) != hipSuccess) return e;
+  SkArgs u{};
+  u.xh = yf; u.B = B; u.N = I; u.K = H; u.ssq = ssq;
+  u.w0 = (const uint16_t*)lw.gate_proj_weight; u.w1 = (const uint16_t*)lw.up_proj_weight; u.mh = bf; u.ldm = I;
+  if ((e = launch_skinny<SK_SILU>(cb, u, st)) != hipSuccess) return e;
+  SkArgs dn{};
+  dn.xh = bf; dn.B = B; dn.N = H; dn.K = I; dn.w0 = (const uint16_t*)lw.down_proj_weight; dn.out = x;
+  dn.norm = next; dn.mh = next ? yf : nullptr; dn.ldm = H; dn.ssq_out = ssq;
+  return launch_skinny<SK_RESID>(cb, dn, st);
+}
 
 struct Work {
   float* x;
@@ -1641,20 +1793,20 @@ struct Work {
   float* part;  // split-K partials of the O and down products [splits][M][H]
   float* qpart; // split-K partials of the QKV or gate/up product on small grids [splits][M][4096 or 2 I]
   float* apart; // the attention's key-range chunk partials (attn_plan)
+  float* ssq;   // short prompts: sums of squares per row and 16 columns of x [H / 16][M]
   u64* keys;
   int32_t* bad;
 };
 
-// Prompts of at most small_m(H) tokens run their products on the skinny kernels (weights as the
-// MFMA A operand, the tokens as up to 4 column blocks); longer ones on 128 x 128 tiles (QKV and
-// gate/up split over K on small grids). Measured on MI355X (same box, ms per prefill, skinny /
-// tiles): 0.6B 24 tokens 1.51 / 1.81, 32 1.65 / 1.87, 33 1.84 / 1.87, 40 1.93 / 1.91, 64 2.39 / 2.01;
-// 1.7B 24 tokens 2.61 / 2.87, 32 2.94 / 2.93, 33 3.29 / 2.94, 48 3.74 / 3.01.
-static int small_m(int H) { return H <= 1024 ? 64 : 32; }
+// Prompts of at most SMALL_M tokens run their products on the skinny kernels (weights as the MFMA A
+// operand, the tokens as up to 8 column blocks); longer ones on 128 x 128 tiles (QKV and gate/up split
+// over K on small grids). Measured on MI355X (same box, ms per prefill, skinny / tiles): 1.7B 33 tokens
+// 1.97 / 2.29, 48 2.02 / 2.36, 64 2.08 / 2.43; 0.6B 64 tokens 1.27 against 1.82 for 65 on tiles.
+constexpr int SMALL_M = 64;
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// K splits of a residual product (O or down, N = H columns) on 128 x 128 tiles for M > small_m(H):
+// K splits of a residual product (O or down, N = H columns) on 128 x 128 tiles for M > SMALL_M:
 // as many as keep the grid within one workgroup per CU (the grid then takes gemm_kernel's deeper
 // pipeline), none from 192 tiles on, at most 8, each K range a whole number of 64-wide steps. The
 // partials are added to the residual by the next norm, in split order; without a split the
@@ -1663,14 +1815,14 @@ static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // 12.36 ms, 1.7B prompt 512 / 1,500 5.95 / 13.04 -> 5.47 / 12.77 ms, 2,048 unchanged.
 static int resid_splits(int H, int M, int K) {
   const int tiles = (H / NT) * ((M + MT - 1) / MT);
-  if (M <= small_m(H) || tiles >= 192) return 1;
+  if (M <= SMALL_M || tiles >= 192) return 1;
   int sp = 256 / tiles;
   sp = sp < 8 ? sp : 8;
   while ((K / KT) % sp != 0) --sp;
   return sp;
 }
 
-// K splits of the QKV or gate/up product (`tiles` 128 x 128 tiles, K = H) for M > small_m(H): on a
+// K splits of the QKV or gate/up product (`tiles` 128 x 128 tiles, K = H) for M > SMALL_M: on a
 // grid of at most 128 tiles, as many as keep it within 256 workgroups (one per CU, on gemm_kernel's
 // deeper pipeline), at most 8, each K range a whole number of 64-wide steps; qkv_post_kernel /
 // silu_post_kernel then add the ranges and do the epilogue the tiles would have fused.
@@ -1682,18 +1834,18 @@ static int small_grid_splits(int tiles, int K) {
   return sp;
 }
 static int qkv_splits(int H, int M) {
-  return M <= small_m(H) ? 1 : small_grid_splits((HQ + 2 * HKV) * D / NT * ((M + MT - 1) / MT), H);
+  return M <= SMALL_M ? 1 : small_grid_splits((HQ + 2 * HKV) * D / NT * ((M + MT - 1) / MT), H);
 }
 static int silu_splits(int H, int I, int M) {
-  return M <= small_m(H) ? 1 : small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
+  return M <= SMALL_M ? 1 : small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
 }
 
 // Workspace layout for M rows: x fp32 [M][H]; a (hi, lo) bf16, max(H, 2048) columns; b (hi, lo)
 // bf16, I columns (a and b: row-major for the skinny kernels, fragment-major for gemm_kernel, rows
-// rounded up to MT); q (hi, lo) bf16 [M][2048]; for M <= small_m(H) the raw Q/K/V sums; the split-K partials of
+// rounded up to MT); q (hi, lo) bf16 [M][2048]; for M <= SMALL_M the raw Q/K/V sums; the split-K partials of
 // the residual products; the argmax keys. Offsets in bytes, each 256-byte aligned.
 struct Layout {
-  size_t x, ah, al, bh, bl, qh, ql, raw, part, qpart, apart, keys, bad, bytes;
+  size_t x, ah, al, bh, bl, qh, ql, raw, part, qpart, apart, ssq, keys, bad, bytes;
 };
 static Layout layout(int H, int I, int M) {
   const size_t A = H > HQ * D ? H : HQ * D;
@@ -1708,16 +1860,17 @@ static Layout layout(int H, int I, int M) {
   L.bl = take(MA * I * 2);
   L.qh = take((size_t)M * HQ * D * 2);
   L.ql = take((size_t)M * HQ * D * 2);
-  const bool small = M <= small_m(H);
+  const bool small = M <= SMALL_M;
   L.raw = take(small ? (size_t)M * (HQ + 2 * HKV) * D * 4 : 0);
   const int so = resid_splits(H, M, HQ * D), sd = resid_splits(H, M, I);
-  const int sp = small ? 3 : (so > sd ? so : sd);
+  const int sp = so > sd ? so : sd;
   L.part = take(sp > 1 ? (size_t)sp * M * H * 4 : 0);
   const int sq = qkv_splits(H, M), su = silu_splits(H, I, M);
   size_t qp = sq > 1 ? (size_t)sq * M * (HQ + 2 * HKV) * D : 0;
   if (su > 1 && (size_t)su * M * 2 * I > qp) qp = (size_t)su * M * 2 * I;
   L.qpart = take(qp * 4);
   L.apart = take(attn_part_slots(M) * 2 * attn_part_rows(M) * APS * 4);
+  L.ssq = take(small ? (size_t)M * (H / 16) * 4 : 0);
   L.keys = take(8);
   L.bad = take(4);
   L.bytes = o;
@@ -1737,6 +1890,7 @@ static Work carve(void* base, const Layout& L) {
   w.part = reinterpret_cast<float*>(p + L.part);
   w.qpart = reinterpret_cast<float*>(p + L.qpart);
   w.apart = reinterpret_cast<float*>(p + L.apart);
+  w.ssq = reinterpret_cast<float*>(p + L.ssq);
   w.keys = reinterpret_cast<u64*>(p + L.keys);
   w.bad = reinterpret_cast<int32_t*>(p + L.bad);
   return w;
@@ -1779,33 +1933,24 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
   MKP_LAUNCH(keys_init_kernel, dim3(1), dim3(64), 0, st, wk.keys, 1, wk.bad);
   const AttnPlan ap = attn_plan(M, position);
   if ((size_t)ap.wgs > attn_part_slots(M)) return hipErrorInvalidValue;  // cannot happen (see attn_plan)
-  const bool small = M <= small_m(H);
+  const bool small = M <= SMALL_M;
   const AttnArgs at0{wk.qh, wk.ql, k_cache, v_cache, wk.ah, wk.al, small ? 2 : 1, M, 0, position, kv, wk.bad,
                      wk.apart, ap.chunk, attn_part_rows(M)};
   const dim3 attn_grid(ap.wgs);
   if (small) {
-    // Short prompts: the products are weight-bandwidth bound, so they run on the skinny kernels (16
-    // weight rows per workgroup, 256 to 384 workgroups), the O and down products split over K into
-    // partials that the next norm adds to the residual in a fixed order.
-    typedef BatchPlan<H, I> BP;
+    // Short prompts: the products are weight-bandwidth bound, so they run on the skinny kernels, the
+    // norms folded into them (SK_RESID).
     const int cb = column_blocks(M);
-    auto skinny = [&](int epi, dim3 grid, const SkArgs& a) { return launch_skinny(epi, cb, grid, a, st); };
-    const dim3 rows(M), nthr(64);  // one row per single-wave workgroup: the rows spread over M CUs
-    // norms into the products' skinny fragments (hi and lo in ah)
-    auto norm = [&](const int32_t* tk, int S, const uint16_t* w) {
-      hipLaunchKernelGGL((bnorm_kernel<H, 2>), rows, nthr, 0, st, wk.x, tk, embed, dims.vocab, wk.bad, wk.part, S,
-                         w, wk.ah, nullptr, 0, M);
-      return hipGetLastError();
-    };
+    // the embedding rows and their whole norm; from then on the products keep x and its norm products
+    MKP_LAUNCH((bnorm_kernel<H, 2>), dim3(M), dim3(64), 0, st, wk.x, tokens, embed, dims.vocab, wk.bad, nullptr, 0,
+               (const uint16_t*)layers[0].norm_weight, wk.al, nullptr, 0, M);
     for (int l = 0; l < dims.num_layers; ++l) {
       const mk_layer_weights& lw = layers[l];
-      if ((e = norm(l == 0 ? tokens : nullptr, l == 0 ? 0 : BP::SD, (const uint16_t*)lw.norm_weight)) != hipSuccess)
-        return e;
       SkArgs q{};
-      q.xh = wk.ah; q.B = M; q.N = (HQ + 2 * HKV) * D; q.K = H;
+      q.xh = wk.al; q.B = M; q.N = (HQ + 2 * HKV) * D; q.K = H; q.ssq = l ? wk.ssq : nullptr;
       q.w0 = (const uint16_t*)lw.q_weight; q.w1 = (const uint16_t*)lw.k_weight; q.w2 = (const uint16_t*)lw.v_weight;
       q.n1 = HQ * D; q.n2 = (HQ + HKV) * D; q.out = wk.raw;
-      if ((e = skinny(SK_RAW, dim3(q.N / 16, 1), q)) != hipSuccess) return e;
+      if ((e = launch_skinny<SK_RAW>(cb, q, st)) != hipSuccess) return e;
       MKP_LAUNCH(qkv_post_kernel, dim3((M * (HQ + 2 * HKV) + 3) / 4), dim3(64), 0, st, wk.raw, 1, M, position,
                  (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab, wk.qh, wk.ql,
                  k_cache, v_cache, l, kv, wk.bad);
@@ -1813,24 +1958,10 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
       at.layer = l;
       MKP_LAUNCH(attn_kernel, attn_grid, dim3(512), 0, st, at);
       if (ap.merge) MKP_LAUNCH(attn_merge_kernel, dim3(ap.merge), dim3(256), 0, st, at);
-      SkArgs o{};
-      o.xh = wk.ah; o.B = M; o.N = H; o.K = HQ * D;
-      o.w0 = (const uint16_t*)lw.o_proj_weight; o.out = wk.part;
-      if ((e = skinny(SK_PART, dim3(H / 16, BP::SO), o)) != hipSuccess) return e;
-      if ((e = norm(nullptr, BP::SO, (const uint16_t*)lw.post_attn_norm_weight)) != hipSuccess) return e;
-      SkArgs u{};
-      u.xh = wk.ah; u.B = M; u.N = I; u.K = H;
-      u.w0 = (const uint16_t*)lw.gate_proj_weight; u.w1 = (const uint16_t*)lw.up_proj_weight;
-      u.mh = wk.bh; u.ldm = I;
-      if ((e = skinny(SK_SILU, dim3(I / 8, 1), u)) != hipSuccess) return e;
-      SkArgs dn{};
-      dn.xh = wk.bh; dn.B = M; dn.N = H; dn.K = I;
-      dn.w0 = (const uint16_t*)lw.down_proj_weight; dn.out = wk.part;
-      if ((e = skinny(SK_PART, dim3(H / 16, BP::SD), dn)) != hipSuccess) return e;
+      if ((e = skinny_mlp<H, I>(lw, l + 1 < dims.num_layers ? (const uint16_t*)layers[l + 1].norm_weight : nullptr, cb,
+                                M, wk.ah, wk.al, wk.bh, wk.x, wk.ssq, st)) != hipSuccess)
+        return e;
     }
-    // the last layer's down partials into the residual (no norm: the LM head normalises its row)
-    MKP_LAUNCH(bnorm_kernel<H>, rows, nthr, 0, st, wk.x, nullptr, embed, dims.vocab, wk.bad, wk.part, BP::SD,
-               nullptr, nullptr, nullptr, A, M);
   }
   // Longer prompts: 128 x 128 tiles with the epilogues fused; the residual products split over K
   // into partials when their tile grid is small (the norm after them adds the partials).
@@ -1978,7 +2109,7 @@ namespace mkp {
 // Workspace: what grows with the batch in either engine first (residual rows, keys, counters, plan),
 // then, from `rest` on, this engine's other areas -- or the persistent engine's, which share the space.
 struct BLayout {
-  size_t x, keys, bad, count, plan, rest, ah, al, af, bf, raw, part, apart, bytes;
+  size_t x, keys, bad, count, plan, rest, ah, al, af, yf, bf, raw, ssq, apart, bytes;
 };
 static BLayout blayout(int H, int I, int B) {
   const size_t A = H > HQ * D ? H : HQ * D;
@@ -1993,10 +2124,11 @@ static BLayout blayout(int H, int I, int B) {
   L.rest = o;
   L.ah = take(frag_rows(B) * A * 2);  // whole row tiles for the LM head's gemm_kernel
   L.al = take(frag_rows(B) * A * 2);
-  L.af = take(skf_elems(B, (int)A) * 2);  // skinny fragments: the QKV, O and gate/up inputs
+  L.af = take(skf_elems(B, (int)A) * 2);  // skinny fragments: the O (and the LM head's) input
+  L.yf = take(skf_elems(B, H) * 2);       // ... the QKV and gate/up inputs
   L.bf = take(skf_elems(B, I) * 2);       // ... and the down input
   L.raw = take((size_t)B * (HQ + 2 * HKV) * D * 4);
-  L.part = take((size_t)3 * B * H * 4);
+  L.ssq = take((size_t)B * (H / 16) * 4);
   L.apart = take((size_t)plan_items(B) * HKV * 2 * APW * 4);
   L.bytes = o;
   if (B <= 2 * MKB_MAX && L.bytes < L.rest + mkb_workspace_bytes()) L.bytes = L.rest + align256(mkb_workspace_bytes());
@@ -2009,7 +2141,6 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
                             const mk_layer_weights* layers, const uint16_t* cos_tab, const uint16_t* sin_tab,
                             uint16_t* k_cache, uint16_t* v_cache, int max_seq, float* logits, int32_t* out_tokens,
                             char* ws, const BLayout& Lo, hipStream_t st) {
-  typedef BatchPlan<H, I> BP;
   const int A = H > HQ * D ? H : HQ * D;
   float* x = reinterpret_cast<float*>(ws + Lo.x);
   uint16_t* ah = reinterpret_cast<uint16_t*>(ws + Lo.ah);
@@ -2017,7 +2148,8 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
   uint16_t* af = reinterpret_cast<uint16_t*>(ws + Lo.af);
   uint16_t* bf = reinterpret_cast<uint16_t*>(ws + Lo.bf);
   float* raw = reinterpret_cast<float*>(ws + Lo.raw);
-  float* part = reinterpret_cast<float*>(ws + Lo.part);
+  uint16_t* yf = reinterpret_cast<uint16_t*>(ws + Lo.yf);
+  float* ssq = reinterpret_cast<float*>(ws + Lo.ssq);
   float* apart = reinterpret_cast<float*>(ws + Lo.apart);
   u64* keys = reinterpret_cast<u64*>(ws + Lo.keys);
   int32_t* bad = reinterpret_cast<int32_t*>(ws + Lo.bad);
@@ -2034,49 +2166,38 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
              plan);
   const int cb = column_blocks(B);
   const dim3 rows(B), nthr(64);  // norms: one row per single-wave workgroup
-  const int so = BP::SO, sd = BP::SD;
+  // the embedding rows and their whole norm; from then on the products keep x and its norm products
+  MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, tokens, embed, dims.vocab, bad, nullptr, 0,
+             (const uint16_t*)layers[0].norm_weight, yf, nullptr, 0, B);
   for (int l = 0; l < L; ++l) {
     const mk_layer_weights& lw = layers[l];
-    // x (embedding, or + the previous layer's down partials) -> input norm, as skinny fragments
-    MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, l == 0 ? tokens : nullptr, embed, dims.vocab, bad,
-               part, l == 0 ? 0 : sd, (const uint16_t*)lw.norm_weight, af, nullptr, 0, B);
     SkArgs q{};
-    q.xh = af; q.B = B; q.N = (HQ + 2 * HKV) * D; q.K = H;
+    q.xh = yf; q.B = B; q.N = (HQ + 2 * HKV) * D; q.K = H; q.ssq = l ? ssq : nullptr;
     q.w0 = (const uint16_t*)lw.q_weight; q.w1 = (const uint16_t*)lw.k_weight; q.w2 = (const uint16_t*)lw.v_weight;
     q.n1 = HQ * D; q.n2 = (HQ + HKV) * D; q.out = raw;
-    if ((e = launch_skinny(SK_RAW, cb, dim3(q.N / 16, 1), q, st)) != hipSuccess) return e;
+    if ((e = launch_skinny<SK_RAW>(cb, q, st)) != hipSuccess) return e;
     const BAttnArgs at{raw, (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab,
                        k_cache, v_cache, L, l, max_seq, B, plan, apart, count, af};
     MKB_LAUNCH(battn_kernel, dim3(plan_items(B) * HKV), dim3(256), 0, st, at);
-    SkArgs o{};
-    o.xh = af; o.B = B; o.N = H; o.K = HQ * D; o.w0 = (const uint16_t*)lw.o_proj_weight; o.out = part;
-    if ((e = launch_skinny(SK_PART, cb, dim3(H / 16, so), o, st)) != hipSuccess) return e;
-    MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, part, so,
-               (const uint16_t*)lw.post_attn_norm_weight, af, nullptr, 0, B);
-    SkArgs u{};
-    u.xh = af; u.B = B; u.N = I; u.K = H;
-    u.w0 = (const uint16_t*)lw.gate_proj_weight; u.w1 = (const uint16_t*)lw.up_proj_weight; u.mh = bf; u.ldm = I;
-    if ((e = launch_skinny(SK_SILU, cb, dim3(I / 8, 1), u, st)) != hipSuccess) return e;
-    SkArgs dn{};
-    dn.xh = bf; dn.B = B; dn.N = H; dn.K = I; dn.w0 = (const uint16_t*)lw.down_proj_weight;
-    dn.out = part;
-    if ((e = launch_skinny(SK_PART, cb, dim3(H / 16, sd), dn, st)) != hipSuccess) return e;
+    if ((e = skinny_mlp<H, I>(lw, l + 1 < L ? (const uint16_t*)layers[l + 1].norm_weight : nullptr, cb, B, af, yf, bf, x,
+                              ssq, st)) != hipSuccess)
+      return e;
   }
-  // the last layer's down partials and the final norm, then the tied LM head as one more skinny
+  // the final norm, then the tied LM head as one more skinny
   // product (vocabulary rows x the B normalised rows: each table byte read once, on the matrix
   // cores) and the greedy keys
   const bool lm_tiles = B > 8 && dims.vocab % NT == 0;
   if (lm_tiles)
-    MKB_LAUNCH((bnorm_kernel<H, 1>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, part, sd,
+    MKB_LAUNCH((bnorm_kernel<H, 1>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, nullptr, 0,
                final_norm, ah, al, A, B);
   else
-    MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, part, sd,
+    MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, nullptr, 0,
                final_norm, af, nullptr, 0, B);
   if (!lm_tiles) {
     SkArgs lmh{};
     lmh.xh = af; lmh.B = B; lmh.N = dims.vocab; lmh.K = H;
     lmh.w0 = lm_head; lmh.n1 = dims.vocab; lmh.n2 = dims.vocab; lmh.out = logits;
-    if ((e = launch_skinny(SK_RAW, cb, dim3(dims.vocab / 16, 1), lmh, st)) != hipSuccess) return e;
+    if ((e = launch_skinny<SK_RAW>(cb, lmh, st)) != hipSuccess) return e;
   } else {
     // beyond one column block the skinny product re-reads every row's activations per 16 table
     // rows; a 128-row tile of the table reads them once per 128 (the B rows are one row tile)
@@ -2122,13 +2243,12 @@ extern "C" hipError_t mk_decode_batch(const mk_model_dims* dims, int batch, cons
                             cos_table, sin_table, k_cache, v_cache, max_seq_len, logits, out_tokens, ws + Lo.rest,
                             stream);
   }
-  // 17-24 sequences (17-32 with the persistent engine forced) where the persistent kernel applies
-  // to their parts: two persistent launches, MKB_MAX sequences and the rest, one after the other on
-  // the stream (each sequence's cache, token, position, logits and greedy token are its own slices,
-  // so the parts are independent calls). Measured on MI355X (0.6B, ms per step, two launches /
-  // layer by layer), context 256: 17 1.41 / 1.48, 20 1.45 / 1.50, 24 1.49 / 1.52, 28 1.65 / 1.58,
-  // 32 1.70 / 1.61; context 1,500: 24 2.10 / 2.19, 28 2.34 / 2.37, 32 2.48 / 2.47.
-  const int two_max = mkb_engine() == 2 ? 2 * MKB_MAX : MKB_MAX + 8;
+  // 17-32 sequences with the persistent engine forced: two persistent launches, MKB_MAX sequences and the
+  // rest, one after the other on the stream (each sequence's cache, token, position, logits and greedy
+  // token are its own slices, so the parts are independent calls). The automatic engine runs them layer
+  // by layer: measured on MI355X (0.6B, us per step, two launches / layer by layer), 17 sequences 1,385 /
+  // 1,109 at context 256 and 1,808 / 1,556 at 1,500, 24 sequences 1,465 / 1,164 and 2,059 / 1,745.
+  const int two_max = mkb_engine() == 2 ? 2 * MKB_MAX : MKB_MAX;
   if (batch > MKB_MAX && batch <= two_max && mkb_applies(dims, MKB_MAX, max_seq_len) &&
       mkb_applies(dims, batch - MKB_MAX, max_seq_len)) {
     const size_t seq_cache = (size_t)dims->num_layers * HKV * max_seq_len * D;  // elements per sequence

@@ -79,6 +79,8 @@ def engine(request):
     ("mini2k", tuple(1 + 97 * i for i in range(20)), 2, 1),
     ("mini2k", (62, 63, 64, 1279, 1280, 1407), 2, 1),     # positions at the edges of key blocks
     ("mini17", (33, 200, 90), 4, 1),
+    ("mini17", tuple(9 + 7 * i for i in range(17)), 1, 1),   # 1.7B width, every other number of column blocks: 4
+    ("mini17", tuple(2 + 3 * i for i in range(33)), 1, 1),   # ... and 8
     ("mini17", tuple(5 + 37 * i for i in range(12)), 2, 1),  # 1.7B width, 12 sequences: register-blocked products
     ("mini", tuple(3 + 11 * i for i in range(20)), 2, 1),  # 20 sequences: 3 column blocks of 8 (of 4)
     ("mini", tuple(3 + 11 * i for i in range(20)), 2, 2),  # 20 sequences: two persistent launches, 16 + 4
@@ -189,6 +191,30 @@ def test_batch_agrees_with_single_sequence_decode_at_0_6b(q06, engine, lengths, 
     print(f"[batch qwen3-0.6b B={B} engine {engine}] {ms * 1e3:.0f} us per batched step, {B / ms * 1e3:.0f} tokens/s",
           flush=True)
     assert sess.kernel.status() == 0
+
+
+@pytest.mark.parametrize("engine", [1], indirect=True)
+@pytest.mark.parametrize("B", [5, 33])
+def test_batch_vocabulary_of_an_odd_number_of_tiles(mini, engine, B):
+    """The LM head as a skinny product over 255 row tiles (a vocabulary that is a multiple of 16 and not
+    of 128): with 8 column blocks a workgroup otherwise takes two tiles. The logits of the full table
+    restricted to those rows, which the same norm and sums give on another kernel (128 x 128 tiles at
+    33 sequences): fp32 sums of 1,024 products in another order, so within 1024 * 2^-24 of the sum of
+    their magnitudes, below 2e-4 here."""
+    n = 255 * 16
+    gen = torch.Generator().manual_seed(6)
+    shape = (B, mini.shape.layers, 8, mini.max_seq, 128)
+    k0 = (torch.randn(shape, generator=gen) * 0.5).to(torch.bfloat16).to(DEV)
+    v0 = (torch.randn(shape, generator=gen) * 0.5).to(torch.bfloat16).to(DEV)
+    t = torch.arange(3, 3 + B, dtype=torch.int32, device=DEV)
+    p = torch.arange(0, 7 * B, 7, dtype=torch.int32, device=DEV)
+    part = mini.embed[:n].contiguous()
+    run = lambda e: mini.kernel.decode_batch(t, p, e, e, mini.final_norm, mini.layers, mini.cos, mini.sin,
+                                             k0.clone(), v0.clone(), mini.max_seq)
+    full, _ = run(mini.embed)
+    logits, toks = run(part)
+    assert (logits - full[:, :n]).abs().max().item() < 2e-4
+    assert toks.tolist() == [restate.argmax_bf16(row) for row in logits.cpu()]
 
 
 @pytest.mark.parametrize("engine", [1, 2], indirect=True)
