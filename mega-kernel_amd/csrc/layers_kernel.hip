@@ -23,7 +23,7 @@
 // are split over K too, into raw sums that qkv_post_kernel / silu_post_kernel finish. The attention
 // takes one query block per workgroup, or key-range chunks of the blocks merged by
 // attn_merge_kernel where the blocks' key chains are uneven against the grid. Prompts of at most
-// SMALL_M tokens run the products on the skinny kernels of the batched decode instead (weights
+// small_m(H) tokens run the products on the skinny kernels of the batched decode instead (weights
 // as the MFMA A operand, activations in its skinny fragment order, the norms folded into the products).
 //
 // Numerics are the decode kernel's (the reference kernel's fp32 design, /root/reference/
@@ -106,22 +106,23 @@ static size_t frag_rows(int M) { return (size_t)(M + MT - 1) / MT * MT; }
 // at 64 sequences that was the skinny products' bound (rocprof at 64 sequences: ~64 L1 accesses per
 // load instruction, TA address stalls). Rows past the batch are never written; their columns of the
 // products are never read.
-// Fragment order: with 2 or 4 column blocks (CB, skf_blocks) K-block major (the CB fragments of one
-// K block adjacent), with 8 column-block major (the K blocks of one column block adjacent). Every
-// workgroup of a product reads the same fragments at about the same time; measured on MI355X at
-// context 256 (layer by layer, per step), 16 / 32 / 64 sequences: column-block major 1744 / 2412 /
-// 2411 us, K-block major 1513 / 1994 / 2596, row order 1544 / 1979 / 2863.
-__host__ __device__ inline int skf_blocks(int B) { return B <= 8 ? 1 : B <= 16 ? 2 : B <= 32 ? 4 : 8; }
+// Fragment order: with up to 4 column blocks K-block major (the blocks' fragments of one K block
+// adjacent), beyond column-block major (the K blocks of one column block adjacent). Every workgroup of a
+// product reads the same fragments at about the same time; measured on MI355X at context 256 (layer by
+// layer, per step), 16 / 32 / 64 sequences: column-block major 1744 / 2412 / 2411 us, K-block major
+// 1513 / 1994 / 2596, row order 1544 / 1979 / 2863.
+__host__ __device__ inline int skf_blocks(int B) { return (B + 7) / 8; }
 __host__ __device__ inline size_t skf_frag(int cb, int kb, int CB, int K) {
-  return CB == 8 ? (size_t)cb * (K >> 5) + kb : (size_t)kb * CB + cb;
+  return CB > 4 ? (size_t)cb * (K >> 5) + kb : (size_t)kb * CB + cb;
 }
 __host__ __device__ inline size_t skf_off(int b, int k, int part, int B, int K) {
   const int cb = b >> 3, li = 2 * (b & 7) + part, kb = k >> 5, lg = (k & 31) >> 3;
   return ((skf_frag(cb, kb, skf_blocks(B), K) * 64 + lg * 16 + li) << 3) + (k & 7);
 }
-// Elements of the skinny fragments of B rows: whole column blocks of the kernel that reads them (1,
-// 2, 4 or 8 blocks of 8 rows), hi and lo.
-__host__ __device__ inline size_t skf_elems(int B, int K) { return (size_t)skf_blocks(B) * 8 * K * 2; }
+// Elements of the skinny fragments of B rows, hi and lo. A product's last column blocks may lie past
+// skf_blocks(B) (its workgroups take equal numbers of blocks, at most 12): those are inside the buffer,
+// and their columns of the product are never read.
+__host__ __device__ inline size_t skf_elems(int B, int K) { return (size_t)(skf_blocks(B) + 11) * 8 * K * 2; }
 
 // EPI_QKV_PART / EPI_SILU_PART: the QKV / gate-up products split over K on small grids, each K range's
 // raw sums into part[blockIdx.z][M][N] (N = 4096 / 2 I, a tile's columns as in EPI_QKV / EPI_SILU);
@@ -1017,7 +1018,7 @@ enum SkEpi { SK_RAW = 0, SK_RESID = 1, SK_SILU = 2 };
 // (SK_RAW, SK_SILU) scales its sums by rs[b]. (The decode kernel splits its norms the same way.)
 struct SkArgs {
   const uint16_t* xh;  // activations as skinny fragments (skf_off: K inputs, hi and lo) of B rows
-  int B, N, K;
+  int B, N, K;  // activation rows, weight rows, inputs
   // SK_RAW: rows [0, n1) of w0, [n1, n2) of w1, [n2, N) of w2 (Q, K, V); SK_RESID: w0; SK_SILU: w0 gate, w1 up
   const uint16_t* w0;
   const uint16_t* w1;
@@ -1035,8 +1036,8 @@ struct SkArgs {
 // A workgroup of W waves takes RT tiles of 16 weight rows (SK_SILU: the 8 gate and 8 up rows of 8
 // intermediates in each) and CB of the column blocks (blocks CB by ..), K split over the waves, each
 // wave's range a multiple of 32 U (checked on the host).
-// The B operand holds column blocks of 8 rows of activations (a decode batch, or up to 64 prompt
-// tokens): column li of block cb is row 8 cb + li / 2, hi (even li) or lo (odd li), read as skinny
+// The B operand holds column blocks of 8 rows of activations (a decode batch, or the tokens of a
+// short prompt): column li of block cb is row 8 cb + li / 2, hi (even li) or lo (odd li), read as skinny
 // fragments (skf_off). The weight fragments of a K chunk stay in registers across the column blocks, a
 // block's activation fragments across the row tiles; the loads of up to 4 blocks are in flight at once.
 //
@@ -1053,7 +1054,7 @@ __global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int c0 = CB * blockIdx.y, b0 = 8 * c0;  // first column block and activation row
-  const int CBT = CB * gridDim.y;               // column blocks of the fragments
+  const int CBT = skf_blocks(g.B);              // column blocks of the fragments
   const int nb = min(g.B - b0, NC);             // activation rows of this workgroup
   // this lane's weight rows: tile rt, rows li % 8 and 8 + li % 8
   const uint16_t* wp[RT][2];
@@ -1211,14 +1212,22 @@ __global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
 }
 
 template <int EPI, int W, int U, int RT, int CB>
-static hipError_t run_skinny(int cbt, const SkArgs& a, hipStream_t st) {
-  const int tiles = a.N / (EPI == SK_SILU ? 8 : 16);
-  if (a.K % (32 * W * U) != 0 || cbt % CB != 0 || tiles % RT != 0) return hipErrorInvalidValue;  // cannot happen
-  hipLaunchKernelGGL((skinny_kernel<EPI, W, U, RT, CB>), dim3(tiles / RT, cbt / CB), dim3(64 * W), 0, st, a);
+static hipError_t run_skinny(const SkArgs& a, hipStream_t st) {
+  const int tiles = a.N / (EPI == SK_SILU ? 8 : 16), blocks = skf_blocks(a.B);
+  if (a.K % (32 * W * U) != 0 || tiles % RT != 0) return hipErrorInvalidValue;  // cannot happen
+  hipLaunchKernelGGL((skinny_kernel<EPI, W, U, RT, CB>), dim3(tiles / RT, (blocks + CB - 1) / CB), dim3(64 * W), 0, st, a);
   return hipGetLastError();
 }
+// run_skinny with CB = cb, LO <= cb <= HI
+template <int EPI, int W, int U, int RT, int LO, int HI>
+static hipError_t run_skinny_cb(int cb, const SkArgs& a, hipStream_t st) {
+  if constexpr (LO < HI) {
+    if (cb > LO) return run_skinny_cb<EPI, W, U, RT, LO + 1, HI>(cb, a, st);
+  }
+  return cb <= LO ? run_skinny<EPI, W, U, RT, LO>(a, st) : hipErrorInvalidValue;  // (never above HI)
+}
 
-// The skinny product for up to 8 * cbt activation rows (cbt: 1, 2, 4 or 8 column blocks).
+// The skinny product for a.B activation rows, n column blocks of 8.
 // Every CU reads its workgroups' weight rows and all the activations of their column blocks through its
 // L1 (64 bytes per clock): at 64 rows the activations are 8 times a 16-row tile's weights. So a launch
 // takes about 256 workgroups, one per CU, and where 16-row tiles alone would give more, or one column
@@ -1233,37 +1242,37 @@ static hipError_t run_skinny(int cbt, const SkArgs& a, hipStream_t st) {
 //   1.7B at 8 / 16 rows QKV 8.0 / 8.5 -> 6.4 / 7.0, O 6.4 / 6.5 -> 5.5 / 5.6, gate/up 15.9 / 16.4 ->
 //   12.5 / 13.2, down 13.6 / 13.3 -> 11.2 / 11.0
 // (an empty launch takes 2.5 us, one that only reads 8 / 24 / 48 MB 2.9 / 5.6 / 9.6 us). Other wave
-// counts and chunk sizes (W 4, 8, 12, 16 x U 2 .. 16) were within 3% of these or slower.
+// counts and chunk sizes (W 4, 8, 12, 16 x U 2 .. 16) were within 3% of these or slower. At 128 / 160 /
+// 192 rows (0.6B): QKV 9.8 / 11.0 / 12.4, O 7.5 / 8.8 / 9.0, gate/up 12.5 / 14.0 / 18.0, down 10.1 /
+// 11.2 / 12.0. n: at most 24 column blocks at the 0.6B width, 12 at 1.7B (small_m).
 template <int EPI>
-static hipError_t launch_skinny(int cbt, const SkArgs& a, hipStream_t st) {
+static hipError_t launch_skinny(const SkArgs& a, hipStream_t st) {
+  const int n = skf_blocks(a.B);
+  const bool wide = a.K > 1024;  // SK_RAW, SK_SILU: the 1.7B width
   if constexpr (EPI == SK_RAW) {
-    if (cbt == 8 && (a.N / 16) % 2 == 0) return run_skinny<EPI, 8, 4, 2, 4>(cbt, a, st);
-    if (a.K <= 1024) {
-      if (cbt == 1) return run_skinny<EPI, 8, 4, 1, 1>(cbt, a, st);
-      if (cbt == 2) return run_skinny<EPI, 8, 4, 1, 2>(cbt, a, st);
-      return run_skinny<EPI, 8, 4, 1, 4>(cbt, a, st);
-    }
-    if (cbt == 1) return run_skinny<EPI, 4, 8, 1, 1>(cbt, a, st);
-    if (cbt == 2) return run_skinny<EPI, 4, 8, 1, 2>(cbt, a, st);
-    return run_skinny<EPI, 4, 8, 1, 4>(cbt, a, st);
+    if (n > 4 && (a.N / 16) % 2 == 0) return run_skinny_cb<EPI, 8, 4, 2, 3, 12>((n + 1) / 2, a, st);
+    if (wide) return run_skinny_cb<EPI, 4, 8, 1, 1, 4>(n < 4 ? n : 4, a, st);
+    return run_skinny_cb<EPI, 8, 4, 1, 1, 4>(n < 4 ? n : 4, a, st);
   } else if constexpr (EPI == SK_RESID) {
-    const int wgs = a.N / 16 * cbt;  // with one column block each
-    if (wgs <= 256) return run_skinny<EPI, 8, 4, 1, 1>(cbt, a, st);
-    if (wgs <= 512) return a.K > 3072 ? run_skinny<EPI, 8, 8, 1, 2>(cbt, a, st) : run_skinny<EPI, 4, 8, 1, 2>(cbt, a, st);
-    return a.K > 3072 ? run_skinny<EPI, 8, 8, 1, 4>(cbt, a, st) : run_skinny<EPI, 4, 8, 1, 4>(cbt, a, st);
+    const int cb = (a.N / 16 * n + 255) / 256;  // column blocks per workgroup of one tile
+    if (cb == 6) return run_skinny<EPI, 8, 4, 2, 3>(a, st);
+    if (cb == 5) return run_skinny<EPI, 4, 8, 1, 5>(a, st);
+    if (cb == 1) return run_skinny<EPI, 8, 4, 1, 1>(a, st);
+    if (a.K > 3072) return run_skinny_cb<EPI, 8, 8, 1, 2, 4>(cb, a, st);
+    return cb == 2 ? run_skinny<EPI, 4, 8, 1, 2>(a, st) : run_skinny_cb<EPI, 8, 4, 1, 3, 4>(cb, a, st);
   } else {
-    if (cbt == 1) return run_skinny<EPI, 4, 8, 1, 1>(cbt, a, st);
-    if (a.K <= 1024) {
-      if (cbt == 2) return run_skinny<EPI, 4, 8, 2, 2>(cbt, a, st);
-      if (cbt == 4) return run_skinny<EPI, 8, 4, 3, 2>(cbt, a, st);
-      return run_skinny<EPI, 8, 4, 3, 4>(cbt, a, st);
+    if (n == 1) return run_skinny<EPI, 4, 8, 1, 1>(a, st);
+    if (wide) {
+      if (n <= 4) return run_skinny_cb<EPI, 4, 8, 3, 2, 4>(n, a, st);
+      if (n <= 8) return run_skinny_cb<EPI, 4, 4, 3, 5, 8>(n, a, st);
+      return run_skinny_cb<EPI, 4, 4, 6, 5, 6>((n + 1) / 2, a, st);
     }
-    if (cbt == 2) return run_skinny<EPI, 4, 8, 3, 2>(cbt, a, st);
-    if (cbt == 4) return run_skinny<EPI, 4, 8, 3, 4>(cbt, a, st);
-    return run_skinny<EPI, 4, 4, 3, 8>(cbt, a, st);
+    if (n == 2) return run_skinny<EPI, 4, 8, 2, 2>(a, st);
+    if (n <= 16) return run_skinny_cb<EPI, 8, 4, 3, 2, 8>((n + 1) / 2, a, st);
+    if (n <= 20) return run_skinny_cb<EPI, 8, 2, 3, 9, 10>((n + 1) / 2, a, st);
+    return run_skinny<EPI, 4, 4, 6, 6>(a, st);
   }
 }
-static int column_blocks(int rows) { return rows <= 8 ? 1 : rows <= 16 ? 2 : rows <= 32 ? 4 : 8; }
 
 // Rows b < B of the residual: with `tokens`, x[b] = embed[tokens[b]] (a token outside [0, vocab)
 // reads row 0 and sets *bad); with `part`, x[b] += sum over s < S of part[s][b] (in order); then,
@@ -1769,21 +1778,21 @@ __global__ void __launch_bounds__(256) battn_kernel(const BAttnArgs a) {
 // with SiLU, down into the residual. af: the attention's output; yf, ssq: the residual's norm products,
 // read and written; next: the next layer's input norm (null: the last layer); bf: the down input.
 template <int H, int I>
-static hipError_t skinny_mlp(const mk_layer_weights& lw, const uint16_t* next, int cb, int B, const uint16_t* af,
+static hipError_t skinny_mlp(const mk_layer_weights& lw, const uint16_t* next, int B, const uint16_t* af,
                              uint16_t* yf, uint16_t* bf, float* x, float* ssq, hipStream_t st) {
   hipError_t e;
   SkArgs o{};
   o.xh = af; o.B = B; o.N = H; o.K = HQ * D; o.w0 = (const uint16_t*)lw.o_proj_weight; o.out = x;
   o.norm = (const uint16_t*)lw.post_attn_norm_weight; o.mh = yf; o.ldm = H; o.ssq_out = ssq;
-  if ((e = launch_skinny<SK_RESID>(cb, o, st)) != hipSuccess) return e;
+  if ((e = launch_skinny<SK_RESID>(o, st)) != hipSuccess) return e;
   SkArgs u{};
   u.xh = yf; u.B = B; u.N = I; u.K = H; u.ssq = ssq;
   u.w0 = (const uint16_t*)lw.gate_proj_weight; u.w1 = (const uint16_t*)lw.up_proj_weight; u.mh = bf; u.ldm = I;
-  if ((e = launch_skinny<SK_SILU>(cb, u, st)) != hipSuccess) return e;
+  if ((e = launch_skinny<SK_SILU>(u, st)) != hipSuccess) return e;
   SkArgs dn{};
   dn.xh = bf; dn.B = B; dn.N = H; dn.K = I; dn.w0 = (const uint16_t*)lw.down_proj_weight; dn.out = x;
   dn.norm = next; dn.mh = next ? yf : nullptr; dn.ldm = H; dn.ssq_out = ssq;
-  return launch_skinny<SK_RESID>(cb, dn, st);
+  return launch_skinny<SK_RESID>(dn, st);
 }
 
 struct Work {
@@ -1798,15 +1807,18 @@ struct Work {
   int32_t* bad;
 };
 
-// Prompts of at most SMALL_M tokens run their products on the skinny kernels (weights as the MFMA A
-// operand, the tokens as up to 8 column blocks); longer ones on 128 x 128 tiles (QKV and gate/up split
-// over K on small grids). Measured on MI355X (same box, ms per prefill, skinny / tiles): 1.7B 33 tokens
-// 1.97 / 2.29, 48 2.02 / 2.36, 64 2.08 / 2.43; 0.6B 64 tokens 1.27 against 1.82 for 65 on tiles.
-constexpr int SMALL_M = 64;
+// Prompts of at most small_m(H) tokens run their products on the skinny kernels (weights as the MFMA A
+// operand, the tokens as column blocks of 8); longer ones on 128 x 128 tiles (QKV and gate/up split over
+// K on small grids). The tiles read fewer bytes per product but need a norm kernel before each of them
+// and a kernel after each K split. Measured on MI355X (same box, ms per prefill, skinny / tiles): 0.6B 65
+// tokens 1.39 / 1.82, 96 1.46 / 1.89, 128 1.66 / 2.02, 131 1.81 / 2.08, 160 1.87 / 2.12, 192 2.04 /
+// 2.18, 193 2.19 / 2.18, 256 2.28 / 2.31; 1.7B 33 1.83 / 2.29, 64 2.09 / 2.43, 80 2.38 / 2.50, 96 2.53 /
+// 2.56, 112 2.70 / 2.68.
+static int small_m(int H) { return H <= 1024 ? 192 : 96; }
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// K splits of a residual product (O or down, N = H columns) on 128 x 128 tiles for M > SMALL_M:
+// K splits of a residual product (O or down, N = H columns) on 128 x 128 tiles for M > small_m(H):
 // as many as keep the grid within one workgroup per CU (the grid then takes gemm_kernel's deeper
 // pipeline), none from 192 tiles on, at most 8, each K range a whole number of 64-wide steps. The
 // partials are added to the residual by the next norm, in split order; without a split the
@@ -1815,14 +1827,14 @@ static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // 12.36 ms, 1.7B prompt 512 / 1,500 5.95 / 13.04 -> 5.47 / 12.77 ms, 2,048 unchanged.
 static int resid_splits(int H, int M, int K) {
   const int tiles = (H / NT) * ((M + MT - 1) / MT);
-  if (M <= SMALL_M || tiles >= 192) return 1;
+  if (M <= small_m(H) || tiles >= 192) return 1;
   int sp = 256 / tiles;
   sp = sp < 8 ? sp : 8;
   while ((K / KT) % sp != 0) --sp;
   return sp;
 }
 
-// K splits of the QKV or gate/up product (`tiles` 128 x 128 tiles, K = H) for M > SMALL_M: on a
+// K splits of the QKV or gate/up product (`tiles` 128 x 128 tiles, K = H) for M > small_m(H): on a
 // grid of at most 128 tiles, as many as keep it within 256 workgroups (one per CU, on gemm_kernel's
 // deeper pipeline), at most 8, each K range a whole number of 64-wide steps; qkv_post_kernel /
 // silu_post_kernel then add the ranges and do the epilogue the tiles would have fused.
@@ -1834,15 +1846,15 @@ static int small_grid_splits(int tiles, int K) {
   return sp;
 }
 static int qkv_splits(int H, int M) {
-  return M <= SMALL_M ? 1 : small_grid_splits((HQ + 2 * HKV) * D / NT * ((M + MT - 1) / MT), H);
+  return M <= small_m(H) ? 1 : small_grid_splits((HQ + 2 * HKV) * D / NT * ((M + MT - 1) / MT), H);
 }
 static int silu_splits(int H, int I, int M) {
-  return M <= SMALL_M ? 1 : small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
+  return M <= small_m(H) ? 1 : small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
 }
 
 // Workspace layout for M rows: x fp32 [M][H]; a (hi, lo) bf16, max(H, 2048) columns; b (hi, lo)
 // bf16, I columns (a and b: row-major for the skinny kernels, fragment-major for gemm_kernel, rows
-// rounded up to MT); q (hi, lo) bf16 [M][2048]; for M <= SMALL_M the raw Q/K/V sums; the split-K partials of
+// rounded up to MT); q (hi, lo) bf16 [M][2048]; for M <= small_m(H) the raw Q/K/V sums; the split-K partials of
 // the residual products; the argmax keys. Offsets in bytes, each 256-byte aligned.
 struct Layout {
   size_t x, ah, al, bh, bl, qh, ql, raw, part, qpart, apart, ssq, keys, bad, bytes;
@@ -1853,14 +1865,14 @@ static Layout layout(int H, int I, int M) {
   size_t o = 0;
   auto take = [&](size_t n) { const size_t r = o; o += align256(n); return r; };
   const size_t MA = frag_rows(M);  // the GEMMs' activation operands hold whole row tiles
+  const bool small = M <= small_m(H);
   L.x = take((size_t)M * H * 4);
-  L.ah = take(MA * A * 2);
-  L.al = take(MA * A * 2);
-  L.bh = take(MA * I * 2);
-  L.bl = take(MA * I * 2);
+  L.ah = take((small ? skf_elems(M, HQ * D) : MA * A) * 2);
+  L.al = take((small ? skf_elems(M, H) : MA * A) * 2);
+  L.bh = take((small ? skf_elems(M, I) : MA * I) * 2);
+  L.bl = take(small ? 0 : MA * I * 2);
   L.qh = take((size_t)M * HQ * D * 2);
   L.ql = take((size_t)M * HQ * D * 2);
-  const bool small = M <= SMALL_M;
   L.raw = take(small ? (size_t)M * (HQ + 2 * HKV) * D * 4 : 0);
   const int so = resid_splits(H, M, HQ * D), sd = resid_splits(H, M, I);
   const int sp = so > sd ? so : sd;
@@ -1933,14 +1945,13 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
   MKP_LAUNCH(keys_init_kernel, dim3(1), dim3(64), 0, st, wk.keys, 1, wk.bad);
   const AttnPlan ap = attn_plan(M, position);
   if ((size_t)ap.wgs > attn_part_slots(M)) return hipErrorInvalidValue;  // cannot happen (see attn_plan)
-  const bool small = M <= SMALL_M;
+  const bool small = M <= small_m(H);
   const AttnArgs at0{wk.qh, wk.ql, k_cache, v_cache, wk.ah, wk.al, small ? 2 : 1, M, 0, position, kv, wk.bad,
                      wk.apart, ap.chunk, attn_part_rows(M)};
   const dim3 attn_grid(ap.wgs);
   if (small) {
     // Short prompts: the products are weight-bandwidth bound, so they run on the skinny kernels, the
     // norms folded into them (SK_RESID).
-    const int cb = column_blocks(M);
     // the embedding rows and their whole norm; from then on the products keep x and its norm products
     MKP_LAUNCH((bnorm_kernel<H, 2>), dim3(M), dim3(64), 0, st, wk.x, tokens, embed, dims.vocab, wk.bad, nullptr, 0,
                (const uint16_t*)layers[0].norm_weight, wk.al, nullptr, 0, M);
@@ -1950,7 +1961,7 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
       q.xh = wk.al; q.B = M; q.N = (HQ + 2 * HKV) * D; q.K = H; q.ssq = l ? wk.ssq : nullptr;
       q.w0 = (const uint16_t*)lw.q_weight; q.w1 = (const uint16_t*)lw.k_weight; q.w2 = (const uint16_t*)lw.v_weight;
       q.n1 = HQ * D; q.n2 = (HQ + HKV) * D; q.out = wk.raw;
-      if ((e = launch_skinny<SK_RAW>(cb, q, st)) != hipSuccess) return e;
+      if ((e = launch_skinny<SK_RAW>(q, st)) != hipSuccess) return e;
       MKP_LAUNCH(qkv_post_kernel, dim3((M * (HQ + 2 * HKV) + 3) / 4), dim3(64), 0, st, wk.raw, 1, M, position,
                  (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab, wk.qh, wk.ql,
                  k_cache, v_cache, l, kv, wk.bad);
@@ -1958,7 +1969,7 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
       at.layer = l;
       MKP_LAUNCH(attn_kernel, attn_grid, dim3(512), 0, st, at);
       if (ap.merge) MKP_LAUNCH(attn_merge_kernel, dim3(ap.merge), dim3(256), 0, st, at);
-      if ((e = skinny_mlp<H, I>(lw, l + 1 < dims.num_layers ? (const uint16_t*)layers[l + 1].norm_weight : nullptr, cb,
+      if ((e = skinny_mlp<H, I>(lw, l + 1 < dims.num_layers ? (const uint16_t*)layers[l + 1].norm_weight : nullptr,
                                 M, wk.ah, wk.al, wk.bh, wk.x, wk.ssq, st)) != hipSuccess)
         return e;
     }
@@ -2164,7 +2175,6 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
   } while (0)
   MKB_LAUNCH(batch_plan_kernel, dim3(1), dim3(64), 0, st, positions, tokens, dims.vocab, max_seq, B, keys, bad, count,
              plan);
-  const int cb = column_blocks(B);
   const dim3 rows(B), nthr(64);  // norms: one row per single-wave workgroup
   // the embedding rows and their whole norm; from then on the products keep x and its norm products
   MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, tokens, embed, dims.vocab, bad, nullptr, 0,
@@ -2175,12 +2185,12 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
     q.xh = yf; q.B = B; q.N = (HQ + 2 * HKV) * D; q.K = H; q.ssq = l ? ssq : nullptr;
     q.w0 = (const uint16_t*)lw.q_weight; q.w1 = (const uint16_t*)lw.k_weight; q.w2 = (const uint16_t*)lw.v_weight;
     q.n1 = HQ * D; q.n2 = (HQ + HKV) * D; q.out = raw;
-    if ((e = launch_skinny<SK_RAW>(cb, q, st)) != hipSuccess) return e;
+    if ((e = launch_skinny<SK_RAW>(q, st)) != hipSuccess) return e;
     const BAttnArgs at{raw, (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab,
                        k_cache, v_cache, L, l, max_seq, B, plan, apart, count, af};
     MKB_LAUNCH(battn_kernel, dim3(plan_items(B) * HKV), dim3(256), 0, st, at);
-    if ((e = skinny_mlp<H, I>(lw, l + 1 < L ? (const uint16_t*)layers[l + 1].norm_weight : nullptr, cb, B, af, yf, bf, x,
-                              ssq, st)) != hipSuccess)
+    if ((e = skinny_mlp<H, I>(lw, l + 1 < L ? (const uint16_t*)layers[l + 1].norm_weight : nullptr, B, af, yf, bf, x, ssq,
+                              st)) != hipSuccess)
       return e;
   }
   // the final norm, then the tied LM head as one more skinny
@@ -2197,7 +2207,7 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
     SkArgs lmh{};
     lmh.xh = af; lmh.B = B; lmh.N = dims.vocab; lmh.K = H;
     lmh.w0 = lm_head; lmh.n1 = dims.vocab; lmh.n2 = dims.vocab; lmh.out = logits;
-    if ((e = launch_skinny<SK_RAW>(cb, lmh, st)) != hipSuccess) return e;
+    if ((e = launch_skinny<SK_RAW>(lmh, st)) != hipSuccess) return e;
   } else {
     // beyond one column block the skinny product re-reads every row's activations per 16 table
     // rows; a 128-row tile of the table reads them once per 128 (the B rows are one row tile)

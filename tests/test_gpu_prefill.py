@@ -65,15 +65,19 @@ def _check_cache(got, want, upto, tag):
 
 @pytest.mark.parametrize("shape_fixture, P", [("mini", 1), ("mini", 24), ("mini", 32), ("mini", 33), ("mini", 64),
                                               ("mini", 65), ("mini", 100), ("mini", 300), ("mini", 9), ("mini17", 7),
-                                              ("mini17", 16), ("mini17", 33), ("mini17", 65), ("mini17", 32),
+                                              ("mini17", 16), ("mini17", 33), ("mini17", 65), ("mini17", 96),
+                                              ("mini17", 97), ("mini", 80), ("mini", 128), ("mini", 131), ("mini", 160),
+                                              ("mini", 161), ("mini", 192), ("mini", 193), ("mini17", 32),
                                               ("mini17", 64), ("mini17", 200), ("mini_4k", 1000),
                                               ("mini_4k", 3000), ("mini17_2k", 1500)])
 def test_prefill_matches_oracle(shape_fixture, P, request):
     """Prefill from an empty cache against ``restate.prefill`` on the same prompt: the last token's
     logits and greedy token, every K/V row written, and nothing written past the prompt. P = 1 has
-    one key; P <= 64 run the skinny products on activations in skinny fragment order (7: 1 column
-    block, 9 and 16: 2, 24 and 32: 4, 33 and 64: 8), P = 65 one 128-row tile (rows past the prompt dead; QKV and gate/up split over K into raw sums that the post kernels
-    finish, the residual products split over K, several K steps in flight), P = 65 two attention
+    one key; P <= 192 at the 0.6B width and P <= 96 at 1.7B run the skinny products on activations in
+    skinny fragment order, column blocks of 8 tokens (7: one, 9 and 16: two, 24 and 32: four, 33: five
+    of six in two workgroups, 192: 24 of six per workgroup), P = 193 and the 1.7B P = 97 the 128-row
+    tiles (rows past the prompt dead; QKV and gate/up split over K into raw sums that the post kernels
+    finish, the residual products split over K, several K steps in flight); P = 65 has two attention
     query blocks, the second with one row; P = 300 spans 5 query blocks of the attention (key-range
     chunks) and 3 row tiles of the products. From 8 row tiles the residual products are placed row tile by row tile on the
     XCDs: P = 1000 (8 row tiles, 4-way K split), P = 3000 at the 0.6B width (24 row tiles, 192
