@@ -23,7 +23,7 @@
 // are split over K too, into raw sums that qkv_post_kernel / silu_post_kernel finish. The attention
 // takes one query block per workgroup, or key-range chunks of the blocks merged by
 // attn_merge_kernel where the blocks' key chains are uneven against the grid. Prompts of at most
-// small_m(H) tokens run the products on the skinny kernels of the batched decode instead (weights
+// small_m tokens run the products on the skinny kernels of the batched decode instead (weights
 // as the MFMA A operand, activations in its skinny fragment order, the norms folded into the products).
 //
 // Numerics are the decode kernel's (the reference kernel's fp32 design, /root/reference/
@@ -1243,19 +1243,21 @@ static hipError_t run_skinny_cb(int cb, const SkArgs& a, hipStream_t st) {
 //   12.5 / 13.2, down 13.6 / 13.3 -> 11.2 / 11.0
 // (an empty launch takes 2.5 us, one that only reads 8 / 24 / 48 MB 2.9 / 5.6 / 9.6 us). Other wave
 // counts and chunk sizes (W 4, 8, 12, 16 x U 2 .. 16) were within 3% of these or slower. At 128 / 160 /
-// 192 rows (0.6B): QKV 9.8 / 11.0 / 12.4, O 7.5 / 8.8 / 9.0, gate/up 12.5 / 14.0 / 18.0, down 10.1 /
-// 11.2 / 12.0. n: at most 24 column blocks at the 0.6B width, 12 at 1.7B (small_m).
+// 192 / 256 rows (0.6B): QKV 9.8 / 11.0 / 12.4 / 14.3, O 7.5 / 8.8 / 9.0 / 10.0, gate/up 12.5 / 14.0 /
+// 18.0 / 21.0, down 10.1 / 11.2 / 12.0 / 12.9. n: at most 32 column blocks at the 0.6B width, 16 at 1.7B
+// (small_prompt).
 template <int EPI>
 static hipError_t launch_skinny(const SkArgs& a, hipStream_t st) {
   const int n = skf_blocks(a.B);
   const bool wide = a.K > 1024;  // SK_RAW, SK_SILU: the 1.7B width
   if constexpr (EPI == SK_RAW) {
+    if (n > 24) return run_skinny_cb<EPI, 8, 2, 4, 7, 8>((n + 3) / 4, a, st);
     if (n > 4 && (a.N / 16) % 2 == 0) return run_skinny_cb<EPI, 8, 4, 2, 3, 12>((n + 1) / 2, a, st);
     if (wide) return run_skinny_cb<EPI, 4, 8, 1, 1, 4>(n < 4 ? n : 4, a, st);
     return run_skinny_cb<EPI, 8, 4, 1, 1, 4>(n < 4 ? n : 4, a, st);
   } else if constexpr (EPI == SK_RESID) {
     const int cb = (a.N / 16 * n + 255) / 256;  // column blocks per workgroup of one tile
-    if (cb == 6) return run_skinny<EPI, 8, 4, 2, 3>(a, st);
+    if (cb > 5) return run_skinny_cb<EPI, 8, 4, 2, 3, 4>((cb + 1) / 2, a, st);
     if (cb == 5) return run_skinny<EPI, 4, 8, 1, 5>(a, st);
     if (cb == 1) return run_skinny<EPI, 8, 4, 1, 1>(a, st);
     if (a.K > 3072) return run_skinny_cb<EPI, 8, 8, 1, 2, 4>(cb, a, st);
@@ -1265,12 +1267,12 @@ static hipError_t launch_skinny(const SkArgs& a, hipStream_t st) {
     if (wide) {
       if (n <= 4) return run_skinny_cb<EPI, 4, 8, 3, 2, 4>(n, a, st);
       if (n <= 8) return run_skinny_cb<EPI, 4, 4, 3, 5, 8>(n, a, st);
-      return run_skinny_cb<EPI, 4, 4, 6, 5, 6>((n + 1) / 2, a, st);
+      return run_skinny_cb<EPI, 4, 4, 6, 5, 8>((n + 1) / 2, a, st);
     }
     if (n == 2) return run_skinny<EPI, 4, 8, 2, 2>(a, st);
-    if (n <= 16) return run_skinny_cb<EPI, 8, 4, 3, 2, 8>((n + 1) / 2, a, st);
-    if (n <= 20) return run_skinny_cb<EPI, 8, 2, 3, 9, 10>((n + 1) / 2, a, st);
-    return run_skinny<EPI, 4, 4, 6, 6>(a, st);
+    if (n <= 14) return run_skinny_cb<EPI, 8, 4, 3, 2, 7>((n + 1) / 2, a, st);
+    if (n <= 20) return run_skinny_cb<EPI, 8, 2, 3, 8, 10>((n + 1) / 2, a, st);
+    return run_skinny_cb<EPI, 4, 4, 6, 6, 8>((n + 3) / 4, a, st);
   }
 }
 
@@ -1419,6 +1421,255 @@ __global__ void __launch_bounds__(64) qkv_post_kernel(const float* raw, int S, i
   } else if (page >= 0) {
     *reinterpret_cast<uint4*>(k_cache + kv_row(kv, layer, hd - HQ, pos, page) + 8 * t) = pack();
   }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Attention of a whole short prompt (position 0, at most 32 NP <= 256 tokens) straight from the raw
+// Q/K/V sums (fp32 [M][4096]): the work of qkv_post_kernel, attn_kernel and its merge in one launch.
+// Workgroup 8 t + h: queries 16 t .. 16 t + 15 of both heads of K/V head h. It normalises and rotates
+// its queries (bf16 hi/lo) and every key up to its last query, rounds the K/V rows to bf16 in LDS as
+// the cache holds them, and writes its own 16 tokens' rows into the cache; recomputing the earlier keys
+// (a row is 128 dims) costs less than a kernel that writes them first. Then wave w takes head w % 2 and
+// the 32-key blocks w / 2 and w / 2 + 4: scores S^T = K . Q^T and P . V as in attn_kernel; the four
+// waves of a head merge through LDS, max first.
+// Bound by its chain of latencies (the sums' loads, two LDS round trips, the output), hence one pass over
+// all keys with every load issued at the start. Measured on MI355X per layer (0.6B), against the three
+// kernels: 32 tokens 2.6 + 8.1 -> 5.5 us, 131 tokens 4.8 + 9.6 + 4.5 -> 9.9 us.
+// ------------------------------------------------------------------------------------------------
+constexpr int SA_MAX = 256;      // (the staged rows fill the LDS of a CU)
+constexpr int SVS = SA_MAX + 4;  // padded V^T row (520 B: 8 modulo 128, as VSP)
+struct ShortAttnArgs {
+  const float* raw;
+  int M, layer;
+  const uint16_t *q_norm, *k_norm, *cos_tab, *sin_tab;
+  uint16_t *k_cache, *v_cache;
+  KvMap kv;
+  int32_t* bad;
+  uint16_t* out;  // skinny fragments (hi and lo) of the O product
+};
+struct ShortAttnSmem {
+  union {
+    struct {
+      uint16_t ks[SA_MAX][KSP];
+      uint16_t vt[D][SVS];
+      uint16_t qs[2][2][16][KSP];  // head, hi/lo, query
+    } in;
+    float acc[8][16][D + 4];
+  };
+  float ml[8][16][2];
+};
+
+template <int NP>
+__global__ void __launch_bounds__(512) short_attn_kernel(const ShortAttnArgs a) {
+  __shared__ __attribute__((aligned(16))) ShortAttnSmem sm;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lg = lane >> 4;
+  const int kvh = blockIdx.x & 7, q0 = 16 * (blockIdx.x >> 3);
+  const int nk = min(q0 + 16, a.M);  // keys that this workgroup needs
+  constexpr int RAW = (HQ + 2 * HKV) * D;
+  struct Row {
+    float4 x, y;
+  };
+  auto ld_row = [&](int m, int col) {
+    const float* p = a.raw + (size_t)m * RAW + col;
+    return Row{*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4)};
+  };
+  auto vals = [](const Row& r, float (&v)[8]) {
+    v[0] = r.x.x; v[1] = r.x.y; v[2] = r.x.z; v[3] = r.x.w; v[4] = r.y.x; v[5] = r.y.y; v[6] = r.y.z; v[7] = r.y.w;
+  };
+  auto tab = [&](const uint16_t* t, int m) { return *reinterpret_cast<const uint4*>(t + (size_t)m * D + 8 * (li & 7)); };
+  auto pack = [](const float (&v)[8]) {
+    return make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+  };
+  // 16 lanes per row, lane li its dims 8 li .. +7. Query rows: 32 (head, query) pairs, one per 16 lanes;
+  // key rows 32 p + 4 w + lg; V: keys 64 i + 2 vp, + 1 at dims 8 vc .. +7 (conflict-free 32-bit writes)
+  const int qi = 4 * w + lg, qm = min(q0 + (qi & 15), a.M - 1);
+  const int vp = lane & 31, vc = 2 * w + (lane >> 5);
+  constexpr int NV = (NP + 1) / 2;
+  const Row rq = ld_row(qm, (2 * kvh + (qi >> 4)) * D + 8 * li);
+  const uint4 qcs = tab(a.cos_tab, qm), qsn = tab(a.sin_tab, qm);
+  Row rk[NP], rv[NV][2];
+  uint4 kcs[NP], ksn[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int m = min(32 * p + 4 * w + lg, nk - 1);
+    rk[p] = ld_row(m, (HQ + kvh) * D + 8 * li);
+    kcs[p] = tab(a.cos_tab, m);
+    ksn[p] = tab(a.sin_tab, m);
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) rv[i][e] = ld_row(min(64 * i + 2 * vp + e, nk - 1), (HQ + HKV + kvh) * D + 8 * vc);
+  float qw[8], kw[8], cs[8], sn[8], v[8];
+  unpack8(*reinterpret_cast<const uint4*>(a.q_norm + 8 * li), qw);
+  unpack8(*reinterpret_cast<const uint4*>(a.k_norm + 8 * li), kw);
+  {
+    vals(rq, v);
+    unpack8(qcs, cs);
+    unpack8(qsn, sn);
+    head_norm_rope(v, qw, cs, sn, li);
+    uint4 hi, lo;
+    split8(v, hi, lo);
+    *reinterpret_cast<uint4*>(&sm.in.qs[qi >> 4][0][qi & 15][8 * li]) = hi;
+    *reinterpret_cast<uint4*>(&sm.in.qs[qi >> 4][1][qi & 15][8 * li]) = lo;
+  }
+  // rows past nk hold row nk - 1 again: finite, masked
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int m = 32 * p + 4 * w + lg;
+    vals(rk[p], v);
+    unpack8(kcs[p], cs);
+    unpack8(ksn[p], sn);
+    head_norm_rope(v, kw, cs, sn, li);
+    const uint4 k = pack(v);
+    *reinterpret_cast<uint4*>(&sm.in.ks[m][8 * li]) = k;
+    if (m >= q0 && m < nk) {  // this workgroup's own tokens
+      const int page = a.kv.bt ? kv_page(a.kv, m, li == 0 ? a.bad : nullptr) : 0;
+      if (page >= 0) *reinterpret_cast<uint4*>(a.k_cache + kv_row(a.kv, a.layer, kvh, m, page) + 8 * li) = k;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    uint32_t x[2][4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int m = 64 * i + 2 * vp + e;
+      vals(rv[i][e], v);
+      const uint4 u = pack(v);
+      x[e][0] = u.x; x[e][1] = u.y; x[e][2] = u.z; x[e][3] = u.w;
+      if (m >= q0 && m < nk) {
+        const int page = a.kv.bt ? kv_page(a.kv, m, nullptr) : 0;
+        if (page >= 0) *reinterpret_cast<uint4*>(a.v_cache + kv_row(a.kv, a.layer, kvh, m, page) + 8 * vc) = u;
+      }
+    }
+    if (64 * i + 2 * vp < 32 * NP) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        *reinterpret_cast<uint32_t*>(&sm.in.vt[8 * vc + 2 * q][64 * i + 2 * vp]) = (x[0][q] & 0xFFFFu) | (x[1][q] << 16);
+        *reinterpret_cast<uint32_t*>(&sm.in.vt[8 * vc + 2 * q + 1][64 * i + 2 * vp]) = (x[0][q] >> 16) | (x[1][q] & 0xFFFF0000u);
+      }
+    }
+  }
+  __syncthreads();
+  // head hh, 32-key blocks b0 and b0 + 4 (those with a key up to the last query)
+  const int hh = w & 1, b0 = w >> 1;
+  constexpr int NB = NP > 4 ? 2 : 1;
+  constexpr float C = ATT_SCALE * 1.4426950408889634f;
+  f32x4 st[NB][2];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) st[i][mb] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  f32x4 acc[8];
+#pragma unroll
+  for (int nb = 0; nb < 8; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float mx = -INFINITY, l = 0.f;
+  if (32 * b0 < nk) {
+    uint4 fq[2][4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      fq[0][s] = *reinterpret_cast<const uint4*>(&sm.in.qs[hh][0][li][32 * s + 8 * lg]);
+      fq[1][s] = *reinterpret_cast<const uint4*>(&sm.in.qs[hh][1][li][32 * s + 8 * lg]);
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int kb = b0 + 4 * i;
+      if (32 * kb < nk) {
+        f32x4 t[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          uint4 fk[2];
+#pragma unroll
+          for (int mb = 0; mb < 2; ++mb)
+            fk[mb] = *reinterpret_cast<const uint4*>(&sm.in.ks[32 * kb + 16 * mb + li][32 * s + 8 * lg]);
+#pragma unroll
+          for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb) t[mb] = mfma(fk[mb], fq[hl][s], t[mb]);
+        }
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            st[i][mb][j] = 32 * kb + 16 * mb + 4 * lg + j > q0 + li ? -INFINITY : t[mb][j];  // causal
+            mx = fmaxf(mx, st[i][mb][j]);
+          }
+      }
+    }
+    mx = xmax32(xmax16(mx));
+    const float mc = mx == -INFINITY ? 0.f : mx * C;  // a query before all of the wave's keys: weights 0
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int kb = b0 + 4 * i;
+      float pw[8];
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          pw[4 * mb + j] = __builtin_amdgcn_exp2f(fmaf(st[i][mb][j], C, -mc));
+          l += pw[4 * mb + j];
+        }
+      if (32 * kb < nk) {
+        uint4 ph, pl;
+        split8(pw, ph, pl);
+        uint4 fv[8];
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) {
+          const uint16_t* vr = &sm.in.vt[16 * nb + li][32 * kb + 4 * lg];
+          const uint2 v0 = *reinterpret_cast<const uint2*>(vr), v1 = *reinterpret_cast<const uint2*>(vr + 16);
+          fv[nb] = make_uint4(v0.x, v0.y, v1.x, v1.y);
+        }
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) acc[nb] = mfma(ph, fv[nb], acc[nb]);
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) acc[nb] = mfma(pl, fv[nb], acc[nb]);
+      }
+    }
+    l = xsum32(xsum16(l));
+  }
+  __syncthreads();  // the staged rows are done with
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) sm.acc[w][4 * lg + j][16 * nb + li] = acc[nb][j];
+  if (lg == 0) { sm.ml[w][li][0] = mx; sm.ml[w][li][1] = l; }
+  __syncthreads();
+  {  // thread: head tid / 256, query (tid / 16) % 16, dims 8 (tid % 16) .. +7
+    const int h = tid >> 8, q = (tid >> 4) & 15, c = 8 * (tid & 15);
+    float M = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) M = fmaxf(M, sm.ml[2 * b + h][q][0]);  // finite: block 0 holds key 0
+    float L = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const float f = __builtin_amdgcn_exp2f((sm.ml[2 * b + h][q][0] - M) * C);
+      L = fmaf(sm.ml[2 * b + h][q][1], f, L);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = fmaf(sm.acc[2 * b + h][q][c + i], f, o[i]);
+    }
+    const float inv = 1.f / L;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] *= inv;
+    const int m = q0 + q, k = (2 * kvh + h) * D + c;
+    if (m < a.M) {
+      uint4 hi, lo;
+      split8(o, hi, lo);
+      *reinterpret_cast<uint4*>(a.out + skf_off(m, k, 0, a.M, HQ * D)) = hi;
+      *reinterpret_cast<uint4*>(a.out + skf_off(m, k, 1, a.M, HQ * D)) = lo;
+    }
+  }
+}
+
+static hipError_t launch_short_attn(const ShortAttnArgs& a, hipStream_t st) {
+  if (a.M > SA_MAX) return hipErrorInvalidValue;  // cannot happen (small_m)
+  const dim3 grid(8 * ((a.M + 15) / 16)), thr(512);
+  if (a.M <= 32) hipLaunchKernelGGL(short_attn_kernel<1>, grid, thr, 0, st, a);
+  else if (a.M <= 64) hipLaunchKernelGGL(short_attn_kernel<2>, grid, thr, 0, st, a);
+  else if (a.M <= 128) hipLaunchKernelGGL(short_attn_kernel<4>, grid, thr, 0, st, a);
+  else if (a.M <= 192) hipLaunchKernelGGL(short_attn_kernel<6>, grid, thr, 0, st, a);
+  else hipLaunchKernelGGL(short_attn_kernel<8>, grid, thr, 0, st, a);
+  return hipGetLastError();
 }
 
 // silu(gate) * up of M rows from the S K-range sums of EPI_SILU_PART (part[S][M][2 I]: tile t's
@@ -1807,18 +2058,20 @@ struct Work {
   int32_t* bad;
 };
 
-// Prompts of at most small_m(H) tokens run their products on the skinny kernels (weights as the MFMA A
-// operand, the tokens as column blocks of 8); longer ones on 128 x 128 tiles (QKV and gate/up split over
-// K on small grids). The tiles read fewer bytes per product but need a norm kernel before each of them
-// and a kernel after each K split. Measured on MI355X (same box, ms per prefill, skinny / tiles): 0.6B 65
-// tokens 1.39 / 1.82, 96 1.46 / 1.89, 128 1.66 / 2.02, 131 1.81 / 2.08, 160 1.87 / 2.12, 192 2.04 /
-// 2.18, 193 2.19 / 2.18, 256 2.28 / 2.31; 1.7B 33 1.83 / 2.29, 64 2.09 / 2.43, 80 2.38 / 2.50, 96 2.53 /
-// 2.56, 112 2.70 / 2.68.
-static int small_m(int H) { return H <= 1024 ? 192 : 96; }
+// Whether a prompt runs its products on the skinny kernels (weights as the MFMA A operand, the tokens as
+// column blocks of 8) instead of on 128 x 128 tiles (QKV and gate/up split over K on small grids). The
+// tiles read fewer bytes per product but need a norm kernel before each of them and a kernel after each K
+// split, and from position 0 the skinny path's attention is one launch (short_attn_kernel). Measured on
+// MI355X (same box, ms per prefill, skinny / tiles), from position 0: 0.6B 65 tokens 1.24 / 1.82, 96 1.34
+// / 1.89, 131 1.61 / 2.08, 192 1.85 / 2.18, 256 2.09 / 2.30; 1.7B 33 1.70 / 2.29, 64 1.93 / 2.43, 96 2.39
+// / 2.56, 128 2.64 / 2.76. With the general attention (a later chunk): 0.6B 192 2.04 / 2.18, 256 2.28 /
+// 2.31; 1.7B 96 2.53 / 2.56, 112 2.70 / 2.68.
+static int small_m(int H, int position) { return H <= 1024 ? 256 : position == 0 ? 128 : 96; }
+static bool small_prompt(int H, int M, int position) { return M <= small_m(H, position); }
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// K splits of a residual product (O or down, N = H columns) on 128 x 128 tiles for M > small_m(H):
+// K splits of a residual product (O or down, N = H columns) on 128 x 128 tiles for a prompt on tiles:
 // as many as keep the grid within one workgroup per CU (the grid then takes gemm_kernel's deeper
 // pipeline), none from 192 tiles on, at most 8, each K range a whole number of 64-wide steps. The
 // partials are added to the residual by the next norm, in split order; without a split the
@@ -1827,14 +2080,14 @@ static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // 12.36 ms, 1.7B prompt 512 / 1,500 5.95 / 13.04 -> 5.47 / 12.77 ms, 2,048 unchanged.
 static int resid_splits(int H, int M, int K) {
   const int tiles = (H / NT) * ((M + MT - 1) / MT);
-  if (M <= small_m(H) || tiles >= 192) return 1;
+  if (tiles >= 192) return 1;
   int sp = 256 / tiles;
   sp = sp < 8 ? sp : 8;
   while ((K / KT) % sp != 0) --sp;
   return sp;
 }
 
-// K splits of the QKV or gate/up product (`tiles` 128 x 128 tiles, K = H) for M > small_m(H): on a
+// K splits of the QKV or gate/up product (`tiles` 128 x 128 tiles, K = H) for a prompt on tiles: on a
 // grid of at most 128 tiles, as many as keep it within 256 workgroups (one per CU, on gemm_kernel's
 // deeper pipeline), at most 8, each K range a whole number of 64-wide steps; qkv_post_kernel /
 // silu_post_kernel then add the ranges and do the epilogue the tiles would have fused.
@@ -1846,26 +2099,25 @@ static int small_grid_splits(int tiles, int K) {
   return sp;
 }
 static int qkv_splits(int H, int M) {
-  return M <= small_m(H) ? 1 : small_grid_splits((HQ + 2 * HKV) * D / NT * ((M + MT - 1) / MT), H);
+  return small_grid_splits((HQ + 2 * HKV) * D / NT * ((M + MT - 1) / MT), H);
 }
 static int silu_splits(int H, int I, int M) {
-  return M <= small_m(H) ? 1 : small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
+  return small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
 }
 
 // Workspace layout for M rows: x fp32 [M][H]; a (hi, lo) bf16, max(H, 2048) columns; b (hi, lo)
 // bf16, I columns (a and b: row-major for the skinny kernels, fragment-major for gemm_kernel, rows
-// rounded up to MT); q (hi, lo) bf16 [M][2048]; for M <= small_m(H) the raw Q/K/V sums; the split-K partials of
+// rounded up to MT); q (hi, lo) bf16 [M][2048]; for a prompt on the skinny kernels the raw Q/K/V sums; the split-K partials of
 // the residual products; the argmax keys. Offsets in bytes, each 256-byte aligned.
 struct Layout {
   size_t x, ah, al, bh, bl, qh, ql, raw, part, qpart, apart, ssq, keys, bad, bytes;
 };
-static Layout layout(int H, int I, int M) {
+static Layout layout(int H, int I, int M, bool small) {
   const size_t A = H > HQ * D ? H : HQ * D;
   Layout L;
   size_t o = 0;
   auto take = [&](size_t n) { const size_t r = o; o += align256(n); return r; };
   const size_t MA = frag_rows(M);  // the GEMMs' activation operands hold whole row tiles
-  const bool small = M <= small_m(H);
   L.x = take((size_t)M * H * 4);
   L.ah = take((small ? skf_elems(M, HQ * D) : MA * A) * 2);
   L.al = take((small ? skf_elems(M, H) : MA * A) * 2);
@@ -1874,10 +2126,10 @@ static Layout layout(int H, int I, int M) {
   L.qh = take((size_t)M * HQ * D * 2);
   L.ql = take((size_t)M * HQ * D * 2);
   L.raw = take(small ? (size_t)M * (HQ + 2 * HKV) * D * 4 : 0);
-  const int so = resid_splits(H, M, HQ * D), sd = resid_splits(H, M, I);
+  const int so = small ? 1 : resid_splits(H, M, HQ * D), sd = small ? 1 : resid_splits(H, M, I);
   const int sp = so > sd ? so : sd;
   L.part = take(sp > 1 ? (size_t)sp * M * H * 4 : 0);
-  const int sq = qkv_splits(H, M), su = silu_splits(H, I, M);
+  const int sq = small ? 1 : qkv_splits(H, M), su = small ? 1 : silu_splits(H, I, M);
   size_t qp = sq > 1 ? (size_t)sq * M * (HQ + 2 * HKV) * D : 0;
   if (su > 1 && (size_t)su * M * 2 * I > qp) qp = (size_t)su * M * 2 * I;
   L.qpart = take(qp * 4);
@@ -1887,6 +2139,11 @@ static Layout layout(int H, int I, int M) {
   L.bad = take(4);
   L.bytes = o;
   return L;
+}
+// Workspace of a call at any position.
+static size_t prefill_bytes(int H, int I, int M) {
+  const size_t s = layout(H, I, M, true).bytes, t = layout(H, I, M, false).bytes;
+  return !small_prompt(H, M, 0) ? t : !small_prompt(H, M, 1) && t > s ? t : s;
 }
 static Work carve(void* base, const Layout& L) {
   char* p = static_cast<char*>(base);
@@ -1945,7 +2202,7 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
   MKP_LAUNCH(keys_init_kernel, dim3(1), dim3(64), 0, st, wk.keys, 1, wk.bad);
   const AttnPlan ap = attn_plan(M, position);
   if ((size_t)ap.wgs > attn_part_slots(M)) return hipErrorInvalidValue;  // cannot happen (see attn_plan)
-  const bool small = M <= small_m(H);
+  const bool small = small_prompt(H, M, position);
   const AttnArgs at0{wk.qh, wk.ql, k_cache, v_cache, wk.ah, wk.al, small ? 2 : 1, M, 0, position, kv, wk.bad,
                      wk.apart, ap.chunk, attn_part_rows(M)};
   const dim3 attn_grid(ap.wgs);
@@ -1962,13 +2219,19 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
       q.w0 = (const uint16_t*)lw.q_weight; q.w1 = (const uint16_t*)lw.k_weight; q.w2 = (const uint16_t*)lw.v_weight;
       q.n1 = HQ * D; q.n2 = (HQ + HKV) * D; q.out = wk.raw;
       if ((e = launch_skinny<SK_RAW>(q, st)) != hipSuccess) return e;
-      MKP_LAUNCH(qkv_post_kernel, dim3((M * (HQ + 2 * HKV) + 3) / 4), dim3(64), 0, st, wk.raw, 1, M, position,
-                 (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab, wk.qh, wk.ql,
-                 k_cache, v_cache, l, kv, wk.bad);
-      AttnArgs at = at0;
-      at.layer = l;
-      MKP_LAUNCH(attn_kernel, attn_grid, dim3(512), 0, st, at);
-      if (ap.merge) MKP_LAUNCH(attn_merge_kernel, dim3(ap.merge), dim3(256), 0, st, at);
+      if (position == 0) {
+        const ShortAttnArgs sa{wk.raw, M, l, (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight,
+                               cos_tab, sin_tab, k_cache, v_cache, kv, wk.bad, wk.ah};
+        if ((e = launch_short_attn(sa, st)) != hipSuccess) return e;
+      } else {
+        MKP_LAUNCH(qkv_post_kernel, dim3((M * (HQ + 2 * HKV) + 3) / 4), dim3(64), 0, st, wk.raw, 1, M, position,
+                   (const uint16_t*)lw.q_norm_weight, (const uint16_t*)lw.k_norm_weight, cos_tab, sin_tab, wk.qh,
+                   wk.ql, k_cache, v_cache, l, kv, wk.bad);
+        AttnArgs at = at0;
+        at.layer = l;
+        MKP_LAUNCH(attn_kernel, attn_grid, dim3(512), 0, st, at);
+        if (ap.merge) MKP_LAUNCH(attn_merge_kernel, dim3(ap.merge), dim3(256), 0, st, at);
+      }
       if ((e = skinny_mlp<H, I>(lw, l + 1 < dims.num_layers ? (const uint16_t*)layers[l + 1].norm_weight : nullptr,
                                 M, wk.ah, wk.al, wk.bh, wk.x, wk.ssq, st)) != hipSuccess)
         return e;
@@ -2049,7 +2312,7 @@ using namespace mkp;
 
 extern "C" size_t mk_prefill_workspace_bytes(const mk_model_dims* dims, int num_tokens) {
   if (!dims || num_tokens < 1) return 0;
-  return layout(dims->hidden, dims->intermediate, num_tokens).bytes;
+  return prefill_bytes(dims->hidden, dims->intermediate, num_tokens);
 }
 
 static hipError_t prefill_impl(const mk_model_dims* dims, const int32_t* tokens, int num_tokens, int position,
@@ -2065,8 +2328,9 @@ static hipError_t prefill_impl(const mk_model_dims* dims, const int32_t* tokens,
   if (!(s06 || s17) || dims->num_layers < 1 || dims->vocab < 1) return hipErrorInvalidValue;
   if (num_tokens < 1 || position < 0 || max_seq_len < 1 || (long long)position + num_tokens > max_seq_len)
     return hipErrorInvalidValue;
-  const Layout L = layout(dims->hidden, dims->intermediate, num_tokens);
-  if (workspace_bytes < L.bytes) return hipErrorInvalidValue;
+  if (workspace_bytes < prefill_bytes(dims->hidden, dims->intermediate, num_tokens)) return hipErrorInvalidValue;
+  const Layout L = layout(dims->hidden, dims->intermediate, num_tokens,
+                          small_prompt(dims->hidden, num_tokens, position));
   const Work wk = carve(workspace, L);
   if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0) return hipErrorInvalidValue;
   const mk_layer_weights* lw = static_cast<const mk_layer_weights*>(layer_weights);  // host array

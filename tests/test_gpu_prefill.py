@@ -66,17 +66,20 @@ def _check_cache(got, want, upto, tag):
 @pytest.mark.parametrize("shape_fixture, P", [("mini", 1), ("mini", 24), ("mini", 32), ("mini", 33), ("mini", 64),
                                               ("mini", 65), ("mini", 100), ("mini", 300), ("mini", 9), ("mini17", 7),
                                               ("mini17", 16), ("mini17", 33), ("mini17", 65), ("mini17", 96),
-                                              ("mini17", 97), ("mini", 80), ("mini", 128), ("mini", 131), ("mini", 160),
-                                              ("mini", 161), ("mini", 192), ("mini", 193), ("mini17", 32),
+                                              ("mini17", 128), ("mini17", 129), ("mini", 80), ("mini", 128), ("mini", 131),
+                                              ("mini", 160),
+                                              ("mini", 161), ("mini", 192), ("mini", 193), ("mini", 225), ("mini", 256),
+                                              ("mini", 257), ("mini17", 32),
                                               ("mini17", 64), ("mini17", 200), ("mini_4k", 1000),
                                               ("mini_4k", 3000), ("mini17_2k", 1500)])
 def test_prefill_matches_oracle(shape_fixture, P, request):
     """Prefill from an empty cache against ``restate.prefill`` on the same prompt: the last token's
     logits and greedy token, every K/V row written, and nothing written past the prompt. P = 1 has
-    one key; P <= 192 at the 0.6B width and P <= 96 at 1.7B run the skinny products on activations in
+    one key; P <= 256 at the 0.6B width and P <= 128 at 1.7B run the skinny products on activations in
     skinny fragment order, column blocks of 8 tokens (7: one, 9 and 16: two, 24 and 32: four, 33: five
-    of six in two workgroups, 192: 24 of six per workgroup), P = 193 and the 1.7B P = 97 the 128-row
-    tiles (rows past the prompt dead; QKV and gate/up split over K into raw sums that the post kernels
+    of six in two workgroups, 192: 24 of six per workgroup), with the attention straight from the
+    products' sums in passes of 32 keys (1, 2, 4, 6 and 8 of them); P = 257 and the 1.7B P = 129 the
+    128-row tiles (rows past the prompt dead; QKV and gate/up split over K into raw sums that the post kernels
     finish, the residual products split over K, several K steps in flight); P = 65 has two attention
     query blocks, the second with one row; P = 300 spans 5 query blocks of the attention (key-range
     chunks) and 3 row tiles of the products. From 8 row tiles the residual products are placed row tile by row tile on the
@@ -101,13 +104,15 @@ def test_prefill_matches_oracle(shape_fixture, P, request):
     assert sess.kernel.status() == 0
 
 
-@pytest.mark.parametrize("shape_fixture, cuts", [("mini", (0, 40, 75, 100)), ("mini_4k", (0, 900, 964, 1000))],
-                         ids=["chunks-40-75", "chunks-900-964"])
+@pytest.mark.parametrize("shape_fixture, cuts", [("mini", (0, 40, 75, 100)), ("mini_4k", (0, 900, 964, 1000)),
+                                                 ("mini17", (0, 100, 196, 300)), ("mini", (0, 3, 250, 510))],
+                         ids=["chunks-40-75", "chunks-900-964", "chunks-100-196-1.7b", "chunks-3-250"])
 def test_prefill_in_chunks_and_decode_after_it(shape_fixture, cuts, request):
     """A prompt fed in three chunks gives the cache and last logits of the one-shot oracle prefill;
     a decode step after it (the decode kernel, reading the prefilled cache) matches the oracle's
     decode step on the oracle's cache. The chunks at 900 and 964 are short prompts (64 and 36
-    tokens) over 16 key blocks each: their attention runs as key-range chunks of one block on 128
+    tokens) over 16 key blocks each (the 1.7B chunks: skinny products from position 0 and, of 96 tokens,
+    from 100, tiles for 104 tokens from 196; the 0.6B ones of 247 and 260 tokens the same): their attention runs as key-range chunks of one block on 128
     workgroups, merged by attn_merge_kernel; the first chunk (900 tokens) as chunks of 4 key
     blocks."""
     mini = request.getfixturevalue(shape_fixture)
