@@ -90,12 +90,12 @@ constexpr int CP = NT + 4;                              // padded fp32 row of th
 // operand of gemm_kernel: 16-row x 32-column blocks of 1 KB, block (m / 16, k / 32) at KB offset
 // (m / 16) * (K / 32) + k / 32; inside a block, MFMA lane l = (m % 16) + 16 * ((k % 32) / 8) holds
 // the 16 bytes of columns [8 ((k % 32) / 8), +8). A wave reads one operand fragment as 1 KB of
-// consecutive bytes. Buffers in this layout hold a multiple of MT rows; rows past M are never
+// consecutive bytes. Buffers in this layout hold a multiple of 2 MT rows (the tallest tile); rows past M are never
 // written, and the sums they produce are never stored.
 __device__ __forceinline__ size_t frag_off(int m, int k, int K) {
   return ((((size_t)(m >> 4) * (K >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (m & 15)) << 3) + (k & 7);
 }
-static size_t frag_rows(int M) { return (size_t)(M + MT - 1) / MT * MT; }
+static size_t frag_rows(int M) { return (size_t)(M + 2 * MT - 1) / (2 * MT) * 2 * MT; }
 
 // Activation operand of the skinny products in fragment order ("skinny fragments", used by the
 // batched decode): for column block cb (sequences 8 cb .. 8 cb + 7) and K block kb (32 inputs), one
@@ -173,21 +173,22 @@ __device__ __forceinline__ const uint16_t* weight_row(const GemmArgs& g, int t, 
   }
 }
 
+template <int NW>
 struct GemmSmem {
   union {
     uint16_t w[NT][KP];
-    float c[MT][CP];
+    float c[32 * NW][CP];
   };
 };
 
-// PF: K steps of operands in flight, loaded ahead in registers. 1: the next step's loads are issued
+// NW: waves (rows of the tile / 32). PF: K steps of operands in flight, loaded ahead in registers. 1: the next step's loads are issued
 // as a step's MFMAs start (two workgroups per CU hide each other's load latency). 4: grids of at
 // most one workgroup per CU (short prompts), where a lone workgroup otherwise waits out most of each
 // load round trip. 2: either. PF 1 and 2 are held to the register budget of two workgroups per CU
 // (256 per lane).
-template <int EPI, int PF = 1>
-__global__ void __launch_bounds__(256, PF == 4 ? 1 : 2) gemm_kernel(const GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) GemmSmem sm;
+template <int EPI, int PF = 1, int NW = 4>
+__global__ void __launch_bounds__(64 * NW, PF == 4 ? 1 : 2) gemm_kernel(const GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) GemmSmem<NW> sm;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int tn = blockIdx.x, tm = blockIdx.y;
   if (gridDim.x <= 16 && gridDim.y >= 8 && (gridDim.x * gridDim.y) % 8 == 0) {
@@ -202,7 +203,7 @@ __global__ void __launch_bounds__(256, PF == 4 ? 1 : 2) gemm_kernel(const GemmAr
     tn = t % gridDim.x;
     tm = t / gridDim.x;
   }
-  const int m0 = tm * MT;
+  const int m0 = tm * 32 * NW;
   const int li = lane & 15, lg = lane >> 4;
   const int kch = g.K >> 5;  // 1 KB fragments per 16-row block
 
@@ -223,18 +224,19 @@ __global__ void __launch_bounds__(256, PF == 4 ? 1 : 2) gemm_kernel(const GemmAr
       }
   };
   // weights: global -> registers -> LDS, 4 chunks of 16 bytes per thread (row c / 8, chunk c % 8)
-  typedef uint4 WStep[4];
+  constexpr int WCH = 16 / NW, NTH = 64 * NW;
+  typedef uint4 WStep[WCH];
   auto load_w = [&](int k0, WStep& rw) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i, row = c >> 3, ch = c & 7;
+    for (int i = 0; i < WCH; ++i) {
+      const int c = tid + NTH * i, row = c >> 3, ch = c & 7;
       rw[i] = ld_stream(reinterpret_cast<const uint4*>(weight_row<EPI>(g, tn, row) + k0 + 8 * ch));
     }
   };
   auto store_w = [&](const WStep& rw) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = tid + 256 * i, row = c >> 3, ch = c & 7;
+    for (int i = 0; i < WCH; ++i) {
+      const int c = tid + NTH * i, row = c >> 3, ch = c & 7;
       *reinterpret_cast<uint4*>(&sm.w[row][8 * ch]) = rw[i];
     }
   };
@@ -2106,8 +2108,8 @@ static int silu_splits(int H, int I, int M) {
 }
 
 // Workspace layout for M rows: x fp32 [M][H]; a (hi, lo) bf16, max(H, 2048) columns; b (hi, lo)
-// bf16, I columns (a and b: row-major for the skinny kernels, fragment-major for gemm_kernel, rows
-// rounded up to MT); q (hi, lo) bf16 [M][2048]; for a prompt on the skinny kernels the raw Q/K/V sums; the split-K partials of
+// bf16, I columns (a and b: skinny fragments for the skinny kernels, fragment-major for gemm_kernel, rows
+// rounded up to 2 MT); q (hi, lo) bf16 [M][2048]; for a prompt on the skinny kernels the raw Q/K/V sums; the split-K partials of
 // the residual products; the argmax keys. Offsets in bytes, each 256-byte aligned.
 struct Layout {
   size_t x, ah, al, bh, bl, qh, ql, raw, part, qpart, apart, ssq, keys, bad, bytes;
@@ -2178,6 +2180,20 @@ static int gemm_pf(dim3 grid, int K) {
 }
 template <int EPI>
 static hipError_t launch_gemm(dim3 grid, const GemmArgs& g, hipStream_t st) {
+  // Between one and two workgroups per CU (half the CUs would take two): 256-row tiles of 8 waves, at most
+  // one per CU, where the epilogue works on whole tiles. Same registers and waves per CU, a third fewer
+  // operand bytes on the busiest CUs. Measured on MI355X: 1.7B prompt 512 gate/up (384 -> 192 workgroups)
+  // 64.7 -> 58.1 us per launch; ms per prefill 1.7B 300 / 400 / 512 tokens 4.17 / 4.51 / 4.68 -> 4.12 /
+  // 4.29 / 4.55, 0.6B 768 / 1,024 / 1,100 / 1,280 / 1,920 3.55 / 3.96 / 4.49 / 4.88 / 5.89 -> 3.48 / 3.89 /
+  // 4.34 / 4.72 / 5.80 (641: 3.35 / 3.37). On grids of 512 or more they are not faster (3,584 tokens QKV
+  // 67.4 / 68.1 us, gate/up 88.9 / 94.6).
+  if constexpr (EPI == EPI_QKV || EPI == EPI_SILU) {
+    const int wgs = (int)(grid.x * grid.y), tall = (int)(grid.x * ((grid.y + 1) / 2));
+    if (grid.z == 1 && wgs > 256 && wgs < 512 && tall <= 256 && g.K / KT % 2 == 0) {
+      hipLaunchKernelGGL((gemm_kernel<EPI, 2, 8>), dim3(grid.x, (grid.y + 1) / 2), dim3(512), 0, st, g);
+      return hipGetLastError();
+    }
+  }
   switch (gemm_pf(grid, g.K)) {
     case 4: hipLaunchKernelGGL((gemm_kernel<EPI, 4>), grid, dim3(256), 0, st, g); break;
     case 2: hipLaunchKernelGGL((gemm_kernel<EPI, 2>), grid, dim3(256), 0, st, g); break;
