@@ -38,6 +38,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "mk_device.h"
 #include "mk_batch.h"
 #include "mk_layers.h"
@@ -832,16 +834,25 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnArgs a) {
   *reinterpret_cast<uint4*>(attn_out(a, m, h * D + 8 * ch, 1)) = lo;
 }
 
-// Chunk plan of the attention over a prompt of M tokens at `position`: chunk = ceil(U / 32) key
-// blocks, U the key blocks of one head's query blocks summed, i.e. about 256 chunk workgroups over
-// the 8 heads (one per CU; a workgroup of attn_kernel fills a CU), when the longest query block has
-// at least 1.25 chunks and 2 key blocks more than one chunk; otherwise no chunks (one workgroup per
-// query block: the grid then holds the work evenly enough, or the merge's extra launch would cost
-// more than the shorter chain saves). Every query block has at most U / chunk + 1 chunks, so the
-// grid holds at most 8 (32 + nqb) workgroups, the size of the partials' area. Measured on MI355X
+// Chunk plan of the attention over a prompt of M tokens at `position`. One workgroup of attn_kernel
+// fills a CU, and workgroup b runs on XCD b % 8, which is K/V head b % 8: each head's chunks go to 32
+// CUs in grid order. The shortest chunk considered is T = ceil(U / 32) key blocks, U the key blocks of
+// one head's query blocks summed (about one chunk per CU). No chunks unless the longest query block has
+// at least 1.25 of those and 2 key blocks more than one of them: the grid otherwise holds the work
+// evenly enough, or the merge's extra launch costs more than the shorter chain saves. Measured on MI355X
 // (0.6B prefill from position 0, same box, against one workgroup per query block): prompt 300 3.11
 // -> 3.05 ms, 512 3.47 -> 3.30, 1024 4.76 -> 4.33, 2048 7.05 -> 6.63; 1.7B 512 6.14 -> 5.92, 1500
 // 12.96 -> 12.60; prompt 100 (2 key blocks) 2.84 -> 2.93 with chunks, hence the 2-block margin.
+// Of T .. T + 5 it takes the chunk whose list schedule ends first: query blocks that are not whole
+// multiples of T leave short chunks over, a few more than there are CUs, and those run as a second round
+// that a slightly longer chunk does not need. A workgroup costs its key blocks and about 2 more (its
+// queries, first loads and partial rows); the merge grows by an eighth of a block per chunk. The sum
+// picked the fastest of T .. T + 5 (to 1%) at each of 11 sizes swept, 0.6B, ms per prefill, T -> picked:
+// 300 tokens at 1,801 2.99 -> 2.81 (5 -> 6 blocks; attention 27.0 -> 20.4 us per launch), 400 at 2,900
+// 3.49 -> 3.32, 64 at 3,000 1.68 -> 1.65, 900 3.85 -> 3.80, 1,500 5.50 -> 5.40, 2,048 6.23 -> 6.19, 3,000
+// 9.57 -> 9.40 (36 -> 40); 300 at 700 and 512 stay at T.
+// Every query block has at most U / chunk + 1 chunks, so the grid holds at most 8 (32 + nqb) workgroups,
+// the size of the partials' area, and a block at most 32 chunks.
 struct AttnPlan {
   int chunk, wgs, merge;  // key blocks per chunk (0: none), attn_kernel and attn_merge_kernel workgroups
 };
@@ -851,13 +862,25 @@ static AttnPlan attn_plan(int M, int position) {
   for (int qb = 0; qb < nqb; ++qb) U += attn_nkb(qb, M, position);
   const int T = (int)((U + 31) / 32), maxn = attn_nkb(nqb - 1, M, position);
   if (4 * maxn < 5 * T || maxn < T + 2) return {0, nqb * HKV, 0};
-  int wgs = 0;
-  for (int c = 0;; ++c) {
-    const int n = attn_round(c, T, M, position, nqb);
-    if (n == 0) break;
-    wgs += n;
+  int chunk = T, wgs = 0;
+  long long best = -1;
+  for (int t = T; t <= T + 5 && maxn >= t + 2; ++t) {
+    long long busy[32] = {};  // per CU of one head's XCD
+    int n, count = 0;
+    for (int c = 0; (n = attn_round(c, t, M, position, nqb)) != 0; ++c, count += n)
+      for (int r = 0; r < n; ++r) {
+        const int left = attn_nkb(nqb - 1 - r, M, position) - c * t;
+        long long* cu = std::min_element(busy, busy + 32);
+        *cu += (left < t ? left : t) + 2;
+      }
+    const long long cost = 8 * *std::max_element(busy, busy + 32) + (maxn + t - 1) / t;
+    if (best < 0 || cost <= best) {
+      best = cost;
+      chunk = t;
+      wgs = count;
+    }
   }
-  return {T, wgs * HKV, attn_round(1, T, M, position, nqb) * HKV * 8};
+  return {chunk, wgs * HKV, attn_round(1, chunk, M, position, nqb) * HKV * 8};
 }
 static size_t attn_part_slots(int M) { return (size_t)HKV * (32 + (M + QB - 1) / QB); }
 static int attn_part_rows(int M) { return M < QB ? M : QB; }

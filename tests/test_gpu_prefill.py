@@ -107,16 +107,17 @@ def test_prefill_matches_oracle(shape_fixture, P, request):
 
 
 @pytest.mark.parametrize("shape_fixture, cuts", [("mini", (0, 40, 75, 100)), ("mini_4k", (0, 900, 964, 1000)),
-                                                 ("mini17", (0, 100, 196, 300)), ("mini", (0, 3, 250, 510))],
-                         ids=["chunks-40-75", "chunks-900-964", "chunks-100-196-1.7b", "chunks-3-250"])
+                                                 ("mini17", (0, 100, 196, 300)), ("mini", (0, 3, 250, 510)),
+                                                 ("mini_4k", (0, 1801, 2101))],
+                         ids=["chunks-40-75", "chunks-900-964", "chunks-100-196-1.7b", "chunks-3-250", "chunks-1801"])
 def test_prefill_in_chunks_and_decode_after_it(shape_fixture, cuts, request):
     """A prompt fed in three chunks gives the cache and last logits of the one-shot oracle prefill;
     a decode step after it (the decode kernel, reading the prefilled cache) matches the oracle's
     decode step on the oracle's cache. The chunks at 900 and 964 are short prompts (64 and 36
     tokens) over 16 key blocks each (the 1.7B chunks: skinny products from position 0 and, of 96 tokens,
-    from 100, tiles for 104 tokens from 196; the 0.6B ones of 247 and 260 tokens the same): their attention runs as key-range chunks of one block on 128
-    workgroups, merged by attn_merge_kernel; the first chunk (900 tokens) as chunks of 4 key
-    blocks."""
+    from 100, tiles for 104 tokens from 196; the 0.6B ones of 247 and 260 tokens the same): their attention runs as key-range chunks of two blocks on 64
+    workgroups, merged by attn_merge_kernel; the first chunk (900 tokens) as chunks of 5 key
+    blocks (of 4 a few short ones would run as a second round), the 300 tokens at 1,801 as chunks of 6."""
     mini = request.getfixturevalue(shape_fixture)
     P = cuts[-1]
     ids = hf.prompt_ids(P, mini.shape.vocab, seed=4)[0].tolist()
