@@ -85,8 +85,8 @@ def test_prefill_matches_oracle(shape_fixture, P, request):
     query blocks, the second with one row; P = 300 spans 5 query blocks of the attention (key-range
     chunks) and 3 row tiles of the products. From 8 row tiles the residual products are placed row tile by row tile on the
     XCDs: P = 1000 (8 row tiles, 4-way K split), P = 3000 at the 0.6B width (24 row tiles, 192
-    tiles: no split, one step in flight) and P = 1500 at the 1.7B width (12 row tiles of 16 column
-    tiles: no split). Grids between one and two workgroups per CU take 256-row tiles: gate/up at P = 1000
+    tiles: no split, two wave groups halving K) and P = 1500 at the 1.7B width (12 row tiles of 16 column
+    tiles: the same). Grids between one and two workgroups per CU take 256-row tiles: gate/up at P = 1000
     and the 1.7B P = 300 (three 128-row tiles in two), QKV at P = 1100."""
     sess = request.getfixturevalue(shape_fixture)
     ids = hf.prompt_ids(P, sess.shape.vocab, seed=3)[0].tolist()
