@@ -2124,7 +2124,7 @@ static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // 12.36 ms, 1.7B prompt 512 / 1,500 5.95 / 13.04 -> 5.47 / 12.77 ms, 2,048 unchanged.
 static int resid_splits(int H, int M, int K) {
   const int tiles = (H / NT) * ((M + MT - 1) / MT);
-  if (tiles >= 192) return 1;
+  if (tiles < 1 || tiles >= 192) return 1;  // (below 1: a shape that no call takes)
   int sp = 256 / tiles;
   sp = sp < 8 ? sp : 8;
   while ((K / KT) % sp != 0) --sp;
@@ -2136,7 +2136,7 @@ static int resid_splits(int H, int M, int K) {
 // deeper pipeline), at most 8, each K range a whole number of 64-wide steps; qkv_post_kernel /
 // silu_post_kernel then add the ranges and do the epilogue the tiles would have fused.
 static int small_grid_splits(int tiles, int K) {
-  if (tiles > 128) return 1;
+  if (tiles < 1 || tiles > 128) return 1;  // (below 1: as resid_splits)
   int sp = 256 / tiles;
   sp = sp < 8 ? sp : 8;
   while ((K / KT) % sp != 0) --sp;

@@ -5,6 +5,8 @@ from CUDA calls). No GPU is used: every call here returns before the first HIP r
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -252,6 +254,22 @@ def test_prefill_entry_point_rejects_bad_arguments_before_launch(lib):
     assert call(nbytes=n1 - 1) == HIP_ERROR_INVALID_VALUE
     assert call(workspace=vp(256 + 16)) == HIP_ERROR_INVALID_VALUE  # not 256-byte aligned
     assert call(workspace=None) == HIP_ERROR_INVALID_VALUE
+
+
+
+@pytest.mark.parametrize("hidden, intermediate", [(64, 3072), (0, 0), (1024, 0), (1024, 32)])
+def test_prefill_workspace_of_an_unsupported_shape_returns(lib, hidden, intermediate):
+    """``mk_prefill_workspace_bytes`` takes any shape (``mk_prefill`` is what refuses it): one narrower than
+    a 128-column tile has no tiles to split, for few tokens as for many. In a child process, since an
+    integer division by zero ends the process."""
+    code = ("import ctypes, sys\n"
+            "lib = ctypes.CDLL(sys.argv[1])\n"
+            "dims = (ctypes.c_int32 * 4)(int(sys.argv[2]), int(sys.argv[3]), 2, 512)\n"
+            "lib.mk_prefill_workspace_bytes.restype = ctypes.c_size_t\n"
+            "assert all(lib.mk_prefill_workspace_bytes(dims, n) > 0 for n in (1, 8, 64, 100, 300, 4000))\n")
+    r = subprocess.run([sys.executable, "-c", code, lib._name, str(hidden), str(intermediate)], capture_output=True,
+                       text=True)
+    assert r.returncode == 0, (r.returncode, r.stderr)
 
 
 
