@@ -133,7 +133,8 @@ hipError_t mk_decode_noalloc(const mk_model_dims* dims, int token_id, const void
  *   layer_weights     HOST array of mk_layer_weights[num_layers] (device pointers inside)
  *   workspace         device memory of at least mk_prefill_workspace_bytes(dims, num_tokens)
  *                     bytes, 256-byte aligned, owned by the caller, not used after the call's work
- *                     completes on `stream`
+ *                     completes on `stream`; the size never shrinks with num_tokens, so the
+ *                     workspace of the longest prompt serves every shorter one
  * A token outside [0, vocab) is embedded as token 0 and the call reports itself as failed in-band
  * (NaN logits, token -1). Asynchronous on `stream`. Argument errors (null pointers, unsupported
  * shape, position + num_tokens > max_seq_len, workspace too small or not 256-byte aligned) return

@@ -257,6 +257,17 @@ def test_prefill_entry_point_rejects_bad_arguments_before_launch(lib):
 
 
 
+@pytest.mark.parametrize("hidden, intermediate", [(1024, 3072), (2048, 6144)])
+def test_prefill_workspace_never_shrinks_with_the_token_count(lib, hidden, intermediate):
+    """A workspace of ``mk_prefill_workspace_bytes(dims, n)`` serves every shorter prompt too (a chunked
+    prompt's ragged last chunk), although fewer tokens can need more room (more K splits, another path)."""
+    dims = (ctypes.c_int32 * 4)(hidden, intermediate, 28, 151936)
+    ws = lib.mk_prefill_workspace_bytes
+    ws.restype, ws.argtypes = ctypes.c_size_t, [ctypes.c_void_p, ctypes.c_int]
+    sizes = [ws(dims, n) for n in range(1, 4200)]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:])), [n + 1 for n in range(4198) if sizes[n] > sizes[n + 1]]
+
+
 @pytest.mark.parametrize("hidden, intermediate", [(64, 3072), (0, 0), (1024, 0), (1024, 32)])
 def test_prefill_workspace_of_an_unsupported_shape_returns(lib, hidden, intermediate):
     """``mk_prefill_workspace_bytes`` takes any shape (``mk_prefill`` is what refuses it): one narrower than
