@@ -92,12 +92,12 @@ constexpr int CP = NT + 4;                              // padded fp32 row of th
 // operand of gemm_kernel: 16-row x 32-column blocks of 1 KB, block (m / 16, k / 32) at KB offset
 // (m / 16) * (K / 32) + k / 32; inside a block, MFMA lane l = (m % 16) + 16 * ((k % 32) / 8) holds
 // the 16 bytes of columns [8 ((k % 32) / 8), +8). A wave reads one operand fragment as 1 KB of
-// consecutive bytes. Buffers in this layout hold a multiple of 2 MT rows (the tallest tile); rows past M are never
+// consecutive bytes. Buffers in this layout hold whole row tiles (operand_rows); rows past M are never
 // written, and the sums they produce are never stored.
 __device__ __forceinline__ size_t frag_off(int m, int k, int K) {
   return ((((size_t)(m >> 4) * (K >> 5) + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (m & 15)) << 3) + (k & 7);
 }
-static size_t frag_rows(int M) { return (size_t)(M + 2 * MT - 1) / (2 * MT) * 2 * MT; }
+static size_t frag_rows(int M) { return (size_t)(M + MT - 1) / MT * MT; }
 
 // Activation operand of the skinny products in fragment order ("skinny fragments", used by the
 // batched decode): for column block cb (sequences 8 cb .. 8 cb + 7) and K block kb (32 inputs), one
@@ -2149,9 +2149,23 @@ static int silu_splits(int H, int I, int M) {
   return small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
 }
 
+// Whether a QKV or gate/up grid of cols x rows 128 x 128 tiles takes 256-row tiles (launch_gemm).
+static bool tall_tiles(int cols, int rows) {
+  return cols * rows > 256 && cols * rows < 512 && cols * ((rows + 1) / 2) <= 256;
+}
+// Rows of the tiles' activation operands: whole row tiles of the tallest product. (256-row tiles for every
+// prompt pad an odd number of 128-row tiles by one more, which moves the operands' hi and lo parts to
+// addresses that are slower to read: 0.6B 257 / 300 / 384 / 576 / 640 tokens 2,430 / 2,467 / 2,590 / 3,033 /
+// 3,082 -> 2,445 / 2,486 / 2,630 / 3,063 / 3,120 us per prefill on MI355X.)
+static size_t operand_rows(int I, int M) {
+  const int rows = (M + MT - 1) / MT;
+  const bool tall = tall_tiles((HQ + 2 * HKV) * D / NT, rows) || tall_tiles(I / (NT / 2), rows);
+  return frag_rows(tall ? (rows + 1) / 2 * 2 * MT : M);
+}
+
 // Workspace layout for M rows: x fp32 [M][H]; a (hi, lo) bf16, max(H, 2048) columns; b (hi, lo)
-// bf16, I columns (a and b: skinny fragments for the skinny kernels, fragment-major for gemm_kernel, rows
-// rounded up to 2 MT); q (hi, lo) bf16 [M][2048]; for a prompt on the skinny kernels the raw Q/K/V sums; the split-K partials of
+// bf16, I columns (a and b: skinny fragments for the skinny kernels, fragment-major for gemm_kernel,
+// operand_rows rows); q (hi, lo) bf16 [M][2048]; for a prompt on the skinny kernels the raw Q/K/V sums; the split-K partials of
 // the residual products; the argmax keys. Offsets in bytes, each 256-byte aligned.
 struct Layout {
   size_t x, ah, al, bh, bl, qh, ql, raw, part, qpart, apart, ssq, keys, bad, bytes;
@@ -2161,7 +2175,7 @@ static Layout layout(int H, int I, int M, bool small) {
   Layout L;
   size_t o = 0;
   auto take = [&](size_t n) { const size_t r = o; o += align256(n); return r; };
-  const size_t MA = frag_rows(M);  // the GEMMs' activation operands hold whole row tiles
+  const size_t MA = operand_rows(I, M);
   L.x = take((size_t)M * H * 4);
   L.ah = take((small ? skf_elems(M, HQ * D) : MA * A) * 2);
   L.al = take((small ? skf_elems(M, H) : MA * A) * 2);
@@ -2241,8 +2255,7 @@ static hipError_t launch_gemm(dim3 grid, const GemmArgs& g, hipStream_t st) {
   // 4.34 / 4.72 / 5.80 (641: 3.35 / 3.37). On grids of 512 or more they are not faster (3,584 tokens QKV
   // 67.4 / 68.1 us, gate/up 88.9 / 94.6).
   if constexpr (EPI == EPI_QKV || EPI == EPI_SILU) {
-    const int wgs = (int)(grid.x * grid.y), tall = (int)(grid.x * ((grid.y + 1) / 2));
-    if (grid.z == 1 && wgs > 256 && wgs < 512 && tall <= 256 && g.K / KT % 2 == 0) {
+    if (grid.z == 1 && tall_tiles((int)grid.x, (int)grid.y) && g.K / KT % 2 == 0) {
       hipLaunchKernelGGL((gemm_kernel<EPI, 2, 8>), dim3(grid.x, (grid.y + 1) / 2), dim3(512), 0, st, g);
       return hipGetLastError();
     }
