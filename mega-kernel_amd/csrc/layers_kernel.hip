@@ -2149,8 +2149,18 @@ static int silu_splits(int H, int I, int M) {
   return small_grid_splits(I / (NT / 2) * ((M + MT - 1) / MT), H);
 }
 
-// Whether a QKV or gate/up grid of cols x rows 128 x 128 tiles takes 256-row tiles (launch_gemm).
-static bool tall_tiles(int cols, int rows) {
+// Whether a QKV or gate/up product of M rows and cols 128-column tiles, not split over K, takes 256-row tiles
+// of 8 waves instead of 128-row ones of 4: between one and two 128-row workgroups per CU (half the CUs would
+// take two), at most one 256-row one. Same registers and waves per CU, a third fewer operand bytes on the
+// busiest CUs. Not for at most 16 rows past a full tile with CUs left over by the full ones: those workgroups
+// have one wave at work and end early. Measured on MI355X, 128 / 256 rows: 1.7B prompt 512 gate/up (384 ->
+// 192 workgroups) 64.7 / 58.1 us per launch; us per prefill 1.7B 272 tokens 4,110 / 4,099, 280 4,131 / 4,095,
+// 384 4,362 / 4,237, 512 4,641 / 4,461; 0.6B 641 3,339 / 3,359, 656 3,341 / 3,360, 660 3,367 / 3,356, 688 3,417
+// / 3,391, 768 3,536 / 3,470, 1,025 4,356 / 4,194, 1,280 4,849 / 4,551, 1,920 5,890 / 5,800. On grids of 512 or
+// more they are not faster (3,584 tokens QKV 67.4 / 68.1 us, gate/up 88.9 / 94.6).
+static bool tall_tiles(int cols, int M) {
+  const int rows = (M + MT - 1) / MT, full = cols * (rows - 1);
+  if (full < 256 && M - (rows - 1) * MT <= 16) return false;
   return cols * rows > 256 && cols * rows < 512 && cols * ((rows + 1) / 2) <= 256;
 }
 // Rows of the tiles' activation operands: whole row tiles of the tallest product. (256-row tiles for every
@@ -2159,7 +2169,7 @@ static bool tall_tiles(int cols, int rows) {
 // 3,082 -> 2,445 / 2,486 / 2,630 / 3,063 / 3,120 us per prefill on MI355X.)
 static size_t operand_rows(int I, int M) {
   const int rows = (M + MT - 1) / MT;
-  const bool tall = tall_tiles((HQ + 2 * HKV) * D / NT, rows) || tall_tiles(I / (NT / 2), rows);
+  const bool tall = tall_tiles((HQ + 2 * HKV) * D / NT, M) || tall_tiles(I / (NT / 2), M);
   return frag_rows(tall ? (rows + 1) / 2 * 2 * MT : M);
 }
 
@@ -2247,15 +2257,8 @@ static int gemm_pf(dim3 grid, int K) {
 }
 template <int EPI>
 static hipError_t launch_gemm(dim3 grid, const GemmArgs& g, hipStream_t st) {
-  // Between one and two workgroups per CU (half the CUs would take two): 256-row tiles of 8 waves, at most
-  // one per CU, where the epilogue works on whole tiles. Same registers and waves per CU, a third fewer
-  // operand bytes on the busiest CUs. Measured on MI355X: 1.7B prompt 512 gate/up (384 -> 192 workgroups)
-  // 64.7 -> 58.1 us per launch; ms per prefill 1.7B 300 / 400 / 512 tokens 4.17 / 4.51 / 4.68 -> 4.12 /
-  // 4.29 / 4.55, 0.6B 768 / 1,024 / 1,100 / 1,280 / 1,920 3.55 / 3.96 / 4.49 / 4.88 / 5.89 -> 3.48 / 3.89 /
-  // 4.34 / 4.72 / 5.80 (641: 3.35 / 3.37). On grids of 512 or more they are not faster (3,584 tokens QKV
-  // 67.4 / 68.1 us, gate/up 88.9 / 94.6).
   if constexpr (EPI == EPI_QKV || EPI == EPI_SILU) {
-    if (grid.z == 1 && tall_tiles((int)grid.x, (int)grid.y) && g.K / KT % 2 == 0) {
+    if (grid.z == 1 && tall_tiles((int)grid.x, g.M) && g.K / KT % 2 == 0) {
       hipLaunchKernelGGL((gemm_kernel<EPI, 2, 8>), dim3(grid.x, (grid.y + 1) / 2), dim3(512), 0, st, g);
       return hipGetLastError();
     }

@@ -72,7 +72,7 @@ def _check_cache(got, want, upto, tag):
                                               ("mini", 257), ("mini17", 32),
                                               ("mini17", 64), ("mini17", 200), ("mini_4k", 1000),
                                               ("mini_4k", 3000), ("mini17_2k", 1500), ("mini_4k", 1100),
-                                              ("mini17_2k", 300)])
+                                              ("mini17_2k", 300), ("mini_4k", 656), ("mini_4k", 657)])
 def test_prefill_matches_oracle(shape_fixture, P, request):
     """Prefill from an empty cache against ``restate.prefill`` on the same prompt: the last token's
     logits and greedy token, every K/V row written, and nothing written past the prompt. P = 1 has
@@ -87,7 +87,8 @@ def test_prefill_matches_oracle(shape_fixture, P, request):
     XCDs: P = 1000 (8 row tiles, 4-way K split), P = 3000 at the 0.6B width (24 row tiles, 192
     tiles: no split, two wave groups halving K) and P = 1500 at the 1.7B width (12 row tiles of 16 column
     tiles: the same). Grids between one and two workgroups per CU take 256-row tiles: gate/up at P = 1000
-    and the 1.7B P = 300 (three 128-row tiles in two), QKV at P = 1100."""
+    and the 1.7B P = 300 (three 128-row tiles in two), QKV at P = 1100;
+    not at most 16 rows past full tiles that leave CUs over: gate/up at P = 656, 256-row tiles at 657."""
     sess = request.getfixturevalue(shape_fixture)
     ids = hf.prompt_ids(P, sess.shape.vocab, seed=3)[0].tolist()
     s = sess.shape
