@@ -108,18 +108,14 @@ static size_t frag_rows(int M) { return (size_t)(M + MT - 1) / MT * MT; }
 // at 64 sequences that was the skinny products' bound (rocprof at 64 sequences: ~64 L1 accesses per
 // load instruction, TA address stalls). Rows past the batch are never written; their columns of the
 // products are never read.
-// Fragment order: with up to 4 column blocks K-block major (the blocks' fragments of one K block
-// adjacent), beyond column-block major (the K blocks of one column block adjacent). Every workgroup of a
-// product reads the same fragments at about the same time; measured on MI355X at context 256 (layer by
-// layer, per step), 16 / 32 / 64 sequences: column-block major 1744 / 2412 / 2411 us, K-block major
-// 1513 / 1994 / 2596, row order 1544 / 1979 / 2863.
+// Column-block major: the K blocks of one column block are adjacent. (K-block major, the column blocks of
+// one K block adjacent, measured on MI355X from 9 to 64 sequences and 16 to 256 prompt tokens at both
+// widths: within 0.4% either way, but 131 tokens 1,612 -> 1,634 us, 40 at 1.7B 1,740 -> 1,754.)
 __host__ __device__ inline int skf_blocks(int B) { return (B + 7) / 8; }
-__host__ __device__ inline size_t skf_frag(int cb, int kb, int CB, int K) {
-  return CB > 4 ? (size_t)cb * (K >> 5) + kb : (size_t)kb * CB + cb;
-}
-__host__ __device__ inline size_t skf_off(int b, int k, int part, int B, int K) {
+__host__ __device__ inline size_t skf_frag(int cb, int kb, int K) { return (size_t)cb * (K >> 5) + kb; }
+__host__ __device__ inline size_t skf_off(int b, int k, int part, int K) {
   const int cb = b >> 3, li = 2 * (b & 7) + part, kb = k >> 5, lg = (k & 31) >> 3;
-  return ((skf_frag(cb, kb, skf_blocks(B), K) * 64 + lg * 16 + li) << 3) + (k & 7);
+  return ((skf_frag(cb, kb, K) * 64 + lg * 16 + li) << 3) + (k & 7);
 }
 // Elements of the skinny fragments of B rows, hi and lo. A product's last column blocks may lie past
 // skf_blocks(B) (its workgroups take equal numbers of blocks, at most 12): those are inside the buffer,
@@ -512,7 +508,7 @@ constexpr int APS = D + 4;  // floats per partial row: acc[128], m, l, pad (16-b
 
 // Where the 8 output values of row m from column k (k % 8 == 0), part 0 (hi) or 1 (lo), go.
 __device__ __forceinline__ uint16_t* attn_out(const AttnArgs& a, int m, int k, int part) {
-  if (a.frag == 2) return a.oh + skf_off(m, k, part, a.M, HQ * D);
+  if (a.frag == 2) return a.oh + skf_off(m, k, part, HQ * D);
   return (part ? a.ol : a.oh) + frag_off(m, k, HQ * D);
 }
 
@@ -1098,7 +1094,6 @@ __global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int c0 = CB * blockIdx.y, b0 = 8 * c0;  // first column block and activation row
-  const int CBT = skf_blocks(g.B);              // column blocks of the fragments
   const int nb = min(g.B - b0, NC);             // activation rows of this workgroup
   // this lane's weight rows: tile rt, rows li % 8 and 8 + li % 8
   const uint16_t* wp[RT][2];
@@ -1146,7 +1141,7 @@ __global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) c[rt][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4* xf = reinterpret_cast<const uint4*>(g.xh) + lane;  // this lane's 16 bytes of fragment 0
-  auto ld_act = [&](int cb, int k) { return xf[skf_frag(c0 + cb, k >> 5, CBT, g.K) * 64]; };
+  auto ld_act = [&](int cb, int k) { return xf[skf_frag(c0 + cb, k >> 5, g.K) * 64]; };
   // R column blocks' activation fragments in flight: block cb + R's loads go into the registers
   // block cb's MFMAs have just read (no copies: a register copy of a pending load would wait for it)
   constexpr int R = CB < 4 ? CB : 4;
@@ -1227,8 +1222,8 @@ __global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
       const float m = gt / (1.f + expf(-gt)) * up;  // silu(gate) * up (/root/reference/megakernel.cu:659-665)
       const uint16_t hi = f32_to_bf16(m), lo = f32_to_bf16(m - bf16_to_f32(hi));
       const int it = 8 * RT * blockIdx.x + i;  // into the down product's skinny fragments (g.ldm inputs)
-      g.mh[skf_off(b0 + b, it, 0, g.B, g.ldm)] = hi;
-      g.mh[skf_off(b0 + b, it, 1, g.B, g.ldm)] = lo;
+      g.mh[skf_off(b0 + b, it, 0, g.ldm)] = hi;
+      g.mh[skf_off(b0 + b, it, 1, g.ldm)] = lo;
     }
   } else if constexpr (EPI == SK_RAW) {
     for (int idx = tid; idx < ROWS * nb; idx += NT) {
@@ -1245,8 +1240,8 @@ __global__ void __launch_bounds__(64 * W) skinny_kernel(const SkArgs g) {
         if (g.mh) {
           const float y = v * nw[i];
           const uint16_t hi = f32_to_bf16(y), lo = f32_to_bf16(y - bf16_to_f32(hi));
-          g.mh[skf_off(b0 + b, n, 0, g.B, g.ldm)] = hi;
-          g.mh[skf_off(b0 + b, n, 1, g.B, g.ldm)] = lo;
+          g.mh[skf_off(b0 + b, n, 0, g.ldm)] = hi;
+          g.mh[skf_off(b0 + b, n, 1, g.ldm)] = lo;
           const float q = row16_sum(v * v);
           if ((r & 15) == 0) g.ssq_out[(size_t)(n >> 4) * g.B + b0 + b] = q;
         }
@@ -1402,8 +1397,8 @@ __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tok
     uint4 hi, lo;
     split8(y, hi, lo);
     if constexpr (LAYOUT == 2) {
-      *reinterpret_cast<uint4*>(ah + skf_off(b, E * lane + k, 0, B, H)) = hi;
-      *reinterpret_cast<uint4*>(ah + skf_off(b, E * lane + k, 1, B, H)) = lo;
+      *reinterpret_cast<uint4*>(ah + skf_off(b, E * lane + k, 0, H)) = hi;
+      *reinterpret_cast<uint4*>(ah + skf_off(b, E * lane + k, 1, H)) = lo;
     } else {
       const size_t o = LAYOUT == 1 ? frag_off(b, E * lane + k, H) : (size_t)b * lda + E * lane + k;
       *reinterpret_cast<uint4*>(ah + o) = hi;
@@ -1699,8 +1694,8 @@ __global__ void __launch_bounds__(512) short_attn_kernel(const ShortAttnArgs a) 
     if (m < a.M) {
       uint4 hi, lo;
       split8(o, hi, lo);
-      *reinterpret_cast<uint4*>(a.out + skf_off(m, k, 0, a.M, HQ * D)) = hi;
-      *reinterpret_cast<uint4*>(a.out + skf_off(m, k, 1, a.M, HQ * D)) = lo;
+      *reinterpret_cast<uint4*>(a.out + skf_off(m, k, 0, HQ * D)) = hi;
+      *reinterpret_cast<uint4*>(a.out + skf_off(m, k, 1, HQ * D)) = lo;
     }
   }
 }
@@ -2061,8 +2056,8 @@ __global__ void __launch_bounds__(256) battn_kernel(const BAttnArgs a) {
     uint4 hi, lo;
     split8(o, hi, lo);
     const int k = (2 * kvh + hh) * D + c;
-    *reinterpret_cast<uint4*>(a.out + skf_off(b, k, 0, a.B, HQ * D)) = hi;
-    *reinterpret_cast<uint4*>(a.out + skf_off(b, k, 1, a.B, HQ * D)) = lo;
+    *reinterpret_cast<uint4*>(a.out + skf_off(b, k, 0, HQ * D)) = hi;
+    *reinterpret_cast<uint4*>(a.out + skf_off(b, k, 1, HQ * D)) = lo;
   }
 }
 
