@@ -1040,12 +1040,12 @@ __global__ void keys_to_tokens_kernel(const u64* keys, int R, const int32_t* bad
 // ------------------------------------------------------------------------------------------------
 // Batched decode: BMAX = 64 sequences at most, one token each per step, every sequence with its own
 // cache ([B][L][8][max_seq][128]) and position. The layer structure of the prefill, with the
-// products as skinny GEMMs: the weights are the MFMA's 16-row operand A and 8 sequences'
-// activations, hi and lo, its 16 columns (B operand column 2b + hl), so one
-// v_mfma_f32_16x16x32_bf16 multiplies 16 weight rows x 32 inputs by 8 sequences at once, up to 8
-// such column blocks per weight fragment, and each weight byte is read once per step. Sums split
-// over K are written as partials and added in a fixed order by the next kernel, so results are
-// deterministic.
+// products as skinny GEMMs (short prompts take them too, up to 256 tokens as rows): the weights are
+// the MFMA's 16-row operand A and 8 rows' activations, hi and lo, its 16 columns (B operand column
+// 2b + hl), so one v_mfma_f32_16x16x32_bf16 multiplies 16 weight rows x 32 inputs by 8 rows at once.
+// A workgroup multiplies a weight fragment by up to 12 such column blocks; with more than it takes,
+// the workgroups of a grid column read the same weight rows. K is split over a workgroup's waves only,
+// their sums added in LDS in a fixed order, so results are deterministic.
 // ------------------------------------------------------------------------------------------------
 constexpr int BMAX = 64;
 
@@ -1266,7 +1266,8 @@ static hipError_t run_skinny_cb(int cb, const SkArgs& a, hipStream_t st) {
   return cb <= LO ? run_skinny<EPI, W, U, RT, LO>(a, st) : hipErrorInvalidValue;  // (never above HI)
 }
 
-// The skinny product for a.B activation rows, n column blocks of 8.
+// The skinny product for a.B activation rows, n column blocks of 8 (at most 32 at the 0.6B width, 16 at 1.7B:
+// small_prompt).
 // Every CU reads its workgroups' weight rows and all the activations of their column blocks through its
 // L1 (64 bytes per clock): at 64 rows the activations are 8 times a 16-row tile's weights. So a launch
 // takes about 256 workgroups, one per CU, and where 16-row tiles alone would give more, or one column
@@ -1280,11 +1281,30 @@ static hipError_t run_skinny_cb(int cb, const SkArgs& a, hipStream_t st) {
 //   6.6 / 6.6 / 7.9;
 //   1.7B at 8 / 16 rows QKV 8.0 / 8.5 -> 6.4 / 7.0, O 6.4 / 6.5 -> 5.5 / 5.6, gate/up 15.9 / 16.4 ->
 //   12.5 / 13.2, down 13.6 / 13.3 -> 11.2 / 11.0
-// (an empty launch takes 2.5 us, one that only reads 8 / 24 / 48 MB 2.9 / 5.6 / 9.6 us). Other wave
-// counts and chunk sizes (W 4, 8, 12, 16 x U 2 .. 16) were within 3% of these or slower. At 128 / 160 /
-// 192 / 256 rows (0.6B): QKV 9.8 / 11.0 / 12.4 / 14.3, O 7.5 / 8.8 / 9.0 / 10.0, gate/up 12.5 / 14.0 /
-// 18.0 / 21.0, down 10.1 / 11.2 / 12.0 / 12.9. n: at most 32 column blocks at the 0.6B width, 16 at 1.7B
-// (small_prompt).
+// (an empty launch takes 2.5 us, one that only reads 8 / 24 / 48 MB 2.9 / 5.6 / 9.6 us).
+// The lines below between W waves, U loads per round and RT tiles, measured the same way (us per launch,
+// the form taken / the other side, at n column blocks):
+//   QKV. Two tiles from n = 5: n 4 one tile 6.0 / 6.2, 5 and 8 two 6.9 and 7.3 / 7.9 and 8.0 (1.7B 4: 8.6 /
+//   9.5, 5 and 8: 10.4 and 11.4 / 12.4 and 12.6). Four from 25: 24 two 12.5 / 13.1, 25 and 32 four 13.9 and
+//   14.4 / 15.0 and 20.5 (1.7B 16: two 14.7 / 16.3). One tile: W 8 U 4 / W 4 U 8 at n 1, 2, 4: 4.6 / 4.5,
+//   5.1 / 4.9, 6.0 / 6.4; K 2,048 (1.7B) is the other way round: W 4 U 8 6.5 / 6.8, 7.1 / 8.1, 8.6 / 9.4.
+//   O and down, by column blocks per workgroup (cb; with one fewer the grid has a second round of
+//   workgroups: cb 2 6.0 / 7.7, 5 8.5 / 12.2). O at 0.6B, W 8 U 4 against W 4 U 8: cb 1 5.2 / 5.4, 2 6.3 / 6.0,
+//   3 6.9 / 7.1, 4 7.6 / 7.8, 5 8.7 / 8.5; two tiles: cb 4 8.0, 5 8.9, 6 9.0 (one tile 9.2), 8 9.8 (10.6). Down
+//   at 0.6B: 6.5 / 7.0, 8.1 / 7.8, 9.0 / 9.1, 9.9 / 10.0, 11.3 / 11.0; two tiles 10.6, 11.9, 11.9 (12.1), 12.8
+//   (14.0). K 6,144 (down at 1.7B): cb 2, 3, 4 W 8 U 8 12.9, 15.1, 16.7 / the faster of the others 13.7, 15.3,
+//   17.1; not at cb 1, 11.4 against W 8 U 4 10.9, nor at 5, 19.4 against 18.7. (At cb 6 there one tile of W 4
+//   U 8 would take 20.2 instead of 21.4.)
+//   Gate/up at 0.6B. n 2 two tiles 5.8 / three 6.5, one 6.3; from 3 three of W 8: n 4 7.1 / two 7.4; U 2 from
+//   15, which keeps 8 column blocks and more in registers: 14 U 4 11.3 / 11.6, 15 and 18 U 2 12.2 and 13.0 /
+//   12.3 and 14.6; six tiles from 21, with a quarter of the blocks each: 32 20.8 / 22.7 (three tiles).
+//   Gate/up at 1.7B. Three tiles from n = 2: 13.0 / one 14.1; U 8 to n = 4 15.6 / 16.0, U 4 from 5: 16.8 /
+//   16.9, 8 19.8 / 20.3; six tiles from 9, with half of the blocks each: 12 and 16 26.8 and 30.7 / 28.9 and 37.2.
+//   Gate/up where another form is the faster one by now: n 1 two tiles (0.6B) or three (1.7B) 5.3 and 11.8
+//   instead of 5.7 and 12.4; 0.6B n 3 two tiles 6.8 instead of 7.2; 0.6B n 21 to 24 three tiles 14.6 to 16.2
+//   instead of 17.8; 1.7B n 9 and 10 three tiles and all blocks 21.5 and 22.8 instead of 25.2 and 25.3.
+// At 128 / 160 / 192 / 256 rows (0.6B): QKV 9.9 / 11.2 / 12.5 / 14.4, O 7.6 / 8.7 / 9.0 / 9.8, gate/up 12.2 /
+// 13.9 / 17.8 / 20.8, down 9.9 / 11.2 / 11.9 / 12.8.
 template <int EPI>
 static hipError_t launch_skinny(const SkArgs& a, hipStream_t st) {
   const int n = skf_blocks(a.B);
@@ -1316,15 +1336,15 @@ static hipError_t launch_skinny(const SkArgs& a, hipStream_t st) {
 }
 
 // Rows b < B of the residual: with `tokens`, x[b] = embed[tokens[b]] (a token outside [0, vocab)
-// reads row 0 and sets *bad); with `part`, x[b] += sum over s < S of part[s][b] (in order); then,
-// with `w`, RMSNorm into the bf16 hi/lo pair in the layout LAYOUT names. One wave per row (any
-// number of waves per workgroup).
-// LAYOUT 0: row order ah/al [B][lda]; 1: the GEMM's fragment order (frag_off, H columns); 2: skinny
-// fragments (skf_off, H inputs, hi and lo both in ah).
-template <int H, int LAYOUT = 0>
+// reads row 0 and sets *bad); with `part`, x[b] += sum over s < S of part[s][b] (in order); then the
+// RMSNorm with weights w as a bf16 hi/lo pair in the layout LAYOUT names. One wave per row (any number
+// of waves per workgroup).
+// LAYOUT 0: no norm, x only (w, ah and al unused); 1: the GEMM's fragment order (frag_off, H columns);
+// 2: skinny fragments (skf_off, H inputs, hi and lo both in ah).
+template <int H, int LAYOUT>
 __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tokens, const uint16_t* embed, int vocab,
                                                     int32_t* bad, const float* part, int S, const uint16_t* w,
-                                                    uint16_t* ah, uint16_t* al, int lda, int B) {
+                                                    uint16_t* ah, uint16_t* al, int B) {
   constexpr int E = H / 64;
   const int lane = threadIdx.x & 63;
   const int b = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -1332,7 +1352,7 @@ __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tok
   // the norm weights first: their loads then overlap the residual's instead of following the
   // reduction (one round trip fewer per call)
   uint4 wr[E / 8];
-  if (w) {
+  if constexpr (LAYOUT != 0) {
 #pragma unroll
     for (int k = 0; k < E; k += 8) wr[k / 8] = *reinterpret_cast<const uint4*>(w + E * lane + k);
   }
@@ -1359,7 +1379,7 @@ __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tok
       v[k] = t.x; v[k + 1] = t.y; v[k + 2] = t.z; v[k + 3] = t.w;
     }
     // the partials in order, four at a time: their loads go out together (one round trip per four
-    // partials instead of one per partial; up to 16 partials come from the batched decode's products)
+    // partials instead of one per partial; at most 8, from the prefill's residual products: resid_splits)
     for (int s0 = 0; s0 < S; s0 += 4) {
       float4 t[4][E / 4];
 #pragma unroll
@@ -1383,7 +1403,7 @@ __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tok
 #pragma unroll
     for (int k = 0; k < E; k += 4) *reinterpret_cast<float4*>(xr + k) = make_float4(v[k], v[k + 1], v[k + 2], v[k + 3]);
   }
-  if (!w) return;
+  if constexpr (LAYOUT == 0) return;
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < E; ++k) ss = fmaf(v[k], v[k], ss);
@@ -1400,7 +1420,7 @@ __global__ void __launch_bounds__(256) bnorm_kernel(float* x, const int32_t* tok
       *reinterpret_cast<uint4*>(ah + skf_off(b, E * lane + k, 0, H)) = hi;
       *reinterpret_cast<uint4*>(ah + skf_off(b, E * lane + k, 1, H)) = lo;
     } else {
-      const size_t o = LAYOUT == 1 ? frag_off(b, E * lane + k, H) : (size_t)b * lda + E * lane + k;
+      const size_t o = frag_off(b, E * lane + k, H);
       *reinterpret_cast<uint4*>(ah + o) = hi;
       *reinterpret_cast<uint4*>(al + o) = lo;
     }
@@ -2104,7 +2124,9 @@ struct Work {
 // MI355X (same box, ms per prefill, skinny / tiles), from position 0: 0.6B 65 tokens 1.24 / 1.82, 96 1.34
 // / 1.89, 131 1.61 / 2.08, 192 1.85 / 2.18, 256 2.09 / 2.30; 1.7B 33 1.70 / 2.29, 64 1.93 / 2.43, 96 2.39
 // / 2.56, 128 2.64 / 2.76. With the general attention (a later chunk): 0.6B 192 2.04 / 2.18, 256 2.28 /
-// 2.31; 1.7B 96 2.53 / 2.56, 112 2.70 / 2.68.
+// 2.31; 1.7B 96 2.53 / 2.56, 97 2.73 / 2.64, 112 2.75 / 2.71, 128 2.84 / 2.78 (at 1,801: 97 2.93 / 2.88, 128
+// 3.06 / 3.01). Those 97-128 tokens are the only prompts whose gate/up is split over K (silu_post_kernel):
+// longer ones have more than 128 tiles.
 static int small_m(int H, int position) { return H <= 1024 ? 256 : position == 0 ? 128 : 96; }
 static bool small_prompt(int H, int M, int position) { return M <= small_m(H, position); }
 
@@ -2283,7 +2305,6 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
                       const uint16_t* lm_head, const uint16_t* final_norm, const mk_layer_weights* layers,
                       const uint16_t* cos_tab, const uint16_t* sin_tab, uint16_t* k_cache, uint16_t* v_cache,
                       const KvMap& kv, float* logits, int32_t* out_token, const Work& wk, hipStream_t st) {
-  const int A = H > HQ * D ? H : HQ * D;
   const int mtiles = (M + MT - 1) / MT;
   hipError_t e;
 #define MKP_LAUNCH(...)                                   \
@@ -2303,7 +2324,7 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
     // norms folded into them (SK_RESID).
     // the embedding rows and their whole norm; from then on the products keep x and its norm products
     MKP_LAUNCH((bnorm_kernel<H, 2>), dim3(M), dim3(64), 0, st, wk.x, tokens, embed, dims.vocab, wk.bad, nullptr, 0,
-               (const uint16_t*)layers[0].norm_weight, wk.al, nullptr, 0, M);
+               (const uint16_t*)layers[0].norm_weight, wk.al, nullptr, M);
     for (int l = 0; l < dims.num_layers; ++l) {
       const mk_layer_weights& lw = layers[l];
       SkArgs q{};
@@ -2342,7 +2363,7 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
     const int nw = M >= 1024 || (H <= 1024 && M >= 512) ? 4 : M >= 512 ? 2 : 1;
     const dim3 rows((M + nw - 1) / nw), nthr(64 * nw);
     MKP_LAUNCH((bnorm_kernel<H, 1>), rows, nthr, 0, st, wk.x, l == 0 ? tokens : nullptr, embed, dims.vocab,
-               wk.bad, wk.part, l > 0 && sd > 1 ? sd : 0, (const uint16_t*)lw.norm_weight, wk.ah, wk.al, A, M);
+               wk.bad, wk.part, l > 0 && sd > 1 ? sd : 0, (const uint16_t*)lw.norm_weight, wk.ah, wk.al, M);
     GemmArgs g{};
     g.ah = wk.ah; g.al = wk.al; g.M = M; g.K = H;
     g.w0 = (const uint16_t*)lw.q_weight; g.w1 = (const uint16_t*)lw.k_weight; g.w2 = (const uint16_t*)lw.v_weight;
@@ -2369,7 +2390,7 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
     go.w0 = (const uint16_t*)lw.o_proj_weight; go.x = wk.x; go.ldx = H; go.part = so > 1 ? wk.part : nullptr;
     if ((e = launch_gemm<EPI_RESID>(dim3(H / NT, mtiles, so), go, st)) != hipSuccess) return e;
     MKP_LAUNCH((bnorm_kernel<H, 1>), rows, nthr, 0, st, wk.x, nullptr, embed, dims.vocab, wk.bad, wk.part,
-               so > 1 ? so : 0, (const uint16_t*)lw.post_attn_norm_weight, wk.ah, wk.al, A, M);
+               so > 1 ? so : 0, (const uint16_t*)lw.post_attn_norm_weight, wk.ah, wk.al, M);
     GemmArgs gu{};
     gu.ah = wk.ah; gu.al = wk.al; gu.M = M; gu.N = 2 * I; gu.K = H;
     gu.w0 = (const uint16_t*)lw.gate_proj_weight; gu.w1 = (const uint16_t*)lw.up_proj_weight;
@@ -2388,8 +2409,8 @@ static hipError_t run(const mk_model_dims& dims, const int32_t* tokens, int M, i
     if ((e = launch_gemm<EPI_RESID>(dim3(H / NT, mtiles, sd), gd, st)) != hipSuccess) return e;
   }
   if (!small && sd > 1)  // the last layer's down partials into the residual
-    MKP_LAUNCH(bnorm_kernel<H>, dim3((M + 3) / 4), dim3(256), 0, st, wk.x, nullptr, embed, dims.vocab, wk.bad, wk.part,
-               sd, nullptr, nullptr, nullptr, A, M);
+    MKP_LAUNCH((bnorm_kernel<H, 0>), dim3((M + 3) / 4), dim3(256), 0, st, wk.x, nullptr, embed, dims.vocab, wk.bad,
+               wk.part, sd, nullptr, nullptr, nullptr, M);
   // the last row's logits and greedy token
   MKP_LAUNCH(lm_head_kernel<H>, dim3(256), dim3(512), 0, st, wk.x, M - 1, final_norm, lm_head, dims.vocab, logits,
              wk.keys, wk.bad);
@@ -2471,8 +2492,6 @@ extern "C" hipError_t mk_prefill_paged(const mk_model_dims* dims, const int32_t*
 // ------------------------------------------------------------------------------------------------
 namespace mkp {
 
-// Split-K factors of the O and down products (each wave's K range a multiple of 256)
-
 // Workspace: what grows with the batch in either engine first (residual rows, keys, counters, plan),
 // then, from `rest` on, this engine's other areas -- or the persistent engine's, which share the space.
 struct BLayout {
@@ -2508,7 +2527,6 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
                             const mk_layer_weights* layers, const uint16_t* cos_tab, const uint16_t* sin_tab,
                             uint16_t* k_cache, uint16_t* v_cache, int max_seq, float* logits, int32_t* out_tokens,
                             char* ws, const BLayout& Lo, hipStream_t st) {
-  const int A = H > HQ * D ? H : HQ * D;
   float* x = reinterpret_cast<float*>(ws + Lo.x);
   uint16_t* ah = reinterpret_cast<uint16_t*>(ws + Lo.ah);
   uint16_t* al = reinterpret_cast<uint16_t*>(ws + Lo.al);
@@ -2534,7 +2552,7 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
   const dim3 rows(B), nthr(64);  // norms: one row per single-wave workgroup
   // the embedding rows and their whole norm; from then on the products keep x and its norm products
   MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, tokens, embed, dims.vocab, bad, nullptr, 0,
-             (const uint16_t*)layers[0].norm_weight, yf, nullptr, 0, B);
+             (const uint16_t*)layers[0].norm_weight, yf, nullptr, B);
   for (int l = 0; l < L; ++l) {
     const mk_layer_weights& lw = layers[l];
     SkArgs q{};
@@ -2555,10 +2573,10 @@ static hipError_t run_batch(const mk_model_dims& dims, int B, const int32_t* tok
   const bool lm_tiles = B > 8 && dims.vocab % NT == 0;
   if (lm_tiles)
     MKB_LAUNCH((bnorm_kernel<H, 1>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, nullptr, 0,
-               final_norm, ah, al, A, B);
+               final_norm, ah, al, B);
   else
     MKB_LAUNCH((bnorm_kernel<H, 2>), rows, nthr, 0, st, x, nullptr, embed, dims.vocab, bad, nullptr, 0,
-               final_norm, af, nullptr, 0, B);
+               final_norm, af, nullptr, B);
   if (!lm_tiles) {
     SkArgs lmh{};
     lmh.xh = af; lmh.B = B; lmh.N = dims.vocab; lmh.K = H;
