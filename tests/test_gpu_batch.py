@@ -79,17 +79,20 @@ def engine(request):
     ("mini2k", tuple(1 + 97 * i for i in range(20)), 2, 1),
     ("mini2k", (62, 63, 64, 1279, 1280, 1407), 2, 1),     # positions at the edges of key blocks
     ("mini17", (33, 200, 90), 4, 1),
-    ("mini17", tuple(9 + 7 * i for i in range(17)), 1, 1),   # 1.7B width, every other number of column blocks: 4
-    ("mini17", tuple(2 + 3 * i for i in range(33)), 1, 1),   # ... and 8
-    ("mini17", tuple(5 + 37 * i for i in range(12)), 2, 1),  # 1.7B width, 12 sequences: register-blocked products
-    ("mini", tuple(3 + 11 * i for i in range(20)), 2, 1),  # 20 sequences: 3 column blocks of 8 (of 4)
+    ("mini17", tuple(9 + 7 * i for i in range(17)), 1, 1),   # 1.7B width, 3 column blocks
+    ("mini17", tuple(4 + 5 * i for i in range(26)), 1, 1),   # ... 4
+    ("mini17", tuple(2 + 3 * i for i in range(33)), 1, 1),   # ... 5
+    ("mini17", tuple(3 + 2 * i for i in range(43)), 1, 1),   # ... 6
+    ("mini17", tuple(1 + 2 * i for i in range(50)), 1, 1),   # ... 7
+    ("mini17", tuple(5 + 37 * i for i in range(12)), 2, 1),  # 1.7B width, 2 column blocks
+    ("mini", tuple(3 + 11 * i for i in range(20)), 2, 1),  # 20 sequences: 3 column blocks of 8
     ("mini", tuple(3 + 11 * i for i in range(20)), 2, 2),  # 20 sequences: two persistent launches, 16 + 4
     ("mini", tuple(1 + 15 * i for i in range(32)), 1, 2),  # 32 sequences: two persistent launches of 16
     ("mini", tuple(1 + 5 * i for i in range(64)), 1, 1),   # the largest batch: 8 column blocks
 ], indirect=["engine"])
 def test_batch_matches_oracle_per_sequence(shape_fixture, lengths, steps, engine, request):
-    """Sequences of different lengths in one batch (so their attention spans 1 to 8 key splits of
-    64, and sequences end a split exactly at 64 and 256): every step, each sequence's logits and
+    """Sequences of different lengths in one batch (so their attention spans 1 to 8 key blocks of
+    64, and sequences end a block exactly at 64 and 256): every step, each sequence's logits and
     greedy token against the restatement on the kernel's cache for that sequence, and its new K/V
     rows. Layer by layer, up to 8 sequences share one 16-column MFMA block; 20 and 64 sequences use 3
     and 8. The persistent kernel (engine 2) runs up to 8 sequences in one column block and up to 16
@@ -259,14 +262,18 @@ def test_persistent_batch_drains_on_request(mini, engine):
     assert torch.isfinite(logits).all() and min(toks.tolist()) >= 0
 
 
-@pytest.mark.parametrize("engine", [2], indirect=True)
-def test_persistent_engine_is_the_one_that_runs(mini, engine):
+@pytest.mark.parametrize("engine, runs", [
+    (2, ((8, True), (16, True), (17, True), (32, True), (33, False))),
+    (0, ((1, True), (16, True), (17, False), (24, False))),
+], indirect=["engine"])
+def test_persistent_engine_is_the_one_that_runs(mini, engine, runs):
     """Engine 2 falls back to the layer-by-layer engine where the persistent kernel does not apply, so
     the other engine-2 cases would pass on the wrong engine if the device check failed. With its phase
     trace on, the persistent kernel stamps every workgroup's kernel start, LM-head start and end (a
     100 MHz counter, in order); the layer-by-layer engine writes nothing there. Checked at 8
     sequences (one MFMA column block), 16 (two) and 17 and 32 (two launches: the trace holds the
-    second one's stamps), and not at 33 (layer by layer)."""
+    second one's stamps), and not at 33 (layer by layer). The automatic engine takes the persistent
+    kernel up to 16 sequences and goes layer by layer from 17 on."""
     import ctypes
 
     from megakernel import build as mkbuild
@@ -275,7 +282,7 @@ def test_persistent_engine_is_the_one_that_runs(mini, engine):
     lib.mk_set_batch_trace.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
     nbytes = lib.mk_batch_trace_bytes()
     maxl, slots, grid = 32, 24, 256
-    for B, persistent in ((8, True), (16, True), (17, True), (32, True), (33, False)):
+    for B, persistent in runs:
         kd = torch.zeros(B, mini.shape.layers, 8, mini.max_seq, 128, dtype=torch.bfloat16, device=DEV)
         vd = torch.zeros_like(kd)
         buf = torch.zeros(nbytes // 8, dtype=torch.int64, device=DEV)

@@ -1,5 +1,6 @@
-"""HIP-graph capture of the multi-kernel entry points: the batched prefill (``prefill``, both of its
-regimes, and at 300 tokens with the attention cut into key-range chunks and merged) and the batched decode (``decode_batch``, the layer-by-layer engine and the persistent
+"""HIP-graph capture of the multi-kernel entry points: the batched prefill (``prefill``: skinny products
+from position 0 and past it, tiles split over K and fused, the attention whole and in key-range chunks that
+are merged) and the batched decode (``decode_batch``, the layer-by-layer engine and the persistent
 kernel), captured with ``torch.cuda.graph`` after an eager call and replayed several times. Between
 replays the test restores the inputs the call mutates (the caches) with eager kernels and runs
 unrelated eager work, then checks every replay bit for bit against the eager result: the graph must
@@ -18,6 +19,16 @@ REPLAYS = 3
 @pytest.fixture(scope="module")
 def mini():
     return Session("mini", 512)
+
+
+@pytest.fixture(scope="module")
+def mini17():
+    return Session("mini-1.7b", 512)
+
+
+@pytest.fixture(scope="module")
+def mini_4k():
+    return Session("mini", 4096)
 
 
 def _capture(fn):
@@ -40,25 +51,36 @@ def _unrelated_eager_work():
     return float((x * 2).sum().item())
 
 
-@pytest.mark.parametrize("P", [24, 100, 300], ids=["skinny-path", "tile-path", "tile-path-key-chunks"])
-def test_prefill_graph_replays_match_eager(mini, P):
+@pytest.mark.parametrize("shape_fixture, P, position", [
+    ("mini", 24, 0), ("mini", 100, 0),     # short_attn_kernel
+    ("mini", 100, 10), ("mini", 100, 60),  # skinny products, qkv_post_kernel, attention whole / in chunks
+    ("mini", 300, 0),                      # tiles, QKV split over K, attention in chunks
+    ("mini17", 104, 10),                   # tiles, QKV and gate/up split over K, attention whole (2 key blocks)
+    ("mini_4k", 1100, 0),                  # 256-row tiles with fused epilogues, attention in chunks
+    ("mini_4k", 3300, 0),                  # fused tiles, O and down unsplit, attention whole (52 key blocks)
+], ids=["skinny-24", "skinny-100", "skinny-at-10", "skinny-at-60-key-chunks", "tiles-split-key-chunks",
+        "tiles-split-1.7b", "tiles-256-rows", "tiles-3300"])
+def test_prefill_graph_replays_match_eager(shape_fixture, P, position, request):
+    mini = request.getfixturevalue(shape_fixture)
     s = mini.shape
     ids = torch.randint(0, s.vocab, (P,), generator=torch.Generator().manual_seed(7), dtype=torch.int64)
     tokens = ids.to(device=DEV, dtype=torch.int32)
-    kd = torch.zeros(s.layers, s.kv_heads, mini.max_seq, s.head_dim, dtype=torch.bfloat16, device=DEV)
-    vd = torch.zeros_like(kd)
+    gen = torch.Generator().manual_seed(8)
+    shape = (s.layers, s.kv_heads, mini.max_seq, s.head_dim)
+    k0, v0 = ((torch.randn(shape, generator=gen) * 0.5).to(torch.bfloat16).to(DEV) for _ in range(2))
+    kd, vd = k0.clone(), v0.clone()
 
     def call():
         return mini.kernel.prefill(tokens, mini.embed, mini.lm_head, mini.final_norm, mini.layers, mini.cos, mini.sin,
-                                   kd, vd, 0, mini.max_seq)
+                                   kd, vd, position, mini.max_seq)
 
     want_logits, want_tok = (t.clone() for t in call())
     want_k, want_v = kd.clone(), vd.clone()
     torch.cuda.synchronize()
     g, (got_logits, got_tok) = _capture(call)
     for r in range(REPLAYS):
-        kd.zero_()
-        vd.zero_()
+        kd.copy_(k0)
+        vd.copy_(v0)
         _unrelated_eager_work()
         torch.cuda.synchronize()
         g.replay()

@@ -63,32 +63,34 @@ def _check_cache(got, want, upto, tag):
     assert rel.max().item() <= 2 ** -8
 
 
-@pytest.mark.parametrize("shape_fixture, P", [("mini", 1), ("mini", 24), ("mini", 32), ("mini", 33), ("mini", 64),
-                                              ("mini", 65), ("mini", 100), ("mini", 300), ("mini", 9), ("mini17", 7),
-                                              ("mini17", 16), ("mini17", 33), ("mini17", 65), ("mini17", 96),
-                                              ("mini17", 128), ("mini17", 129), ("mini", 80), ("mini", 128), ("mini", 131),
-                                              ("mini", 160),
-                                              ("mini", 161), ("mini", 192), ("mini", 193), ("mini", 225), ("mini", 256),
-                                              ("mini", 257), ("mini17", 32),
-                                              ("mini17", 64), ("mini17", 200), ("mini_4k", 1000),
-                                              ("mini_4k", 3000), ("mini17_2k", 1500), ("mini_4k", 1100),
-                                              ("mini17_2k", 300), ("mini_4k", 656), ("mini_4k", 657)])
+# Prompt lengths by the path that they take from position 0 (mini: the 0.6B width, mini17: 1.7B).
+# Skinny products on column blocks of 8 tokens (their number in brackets), the attention straight from their
+# sums in the passes of 32 keys that the line names.
+SKINNY = [
+    *(("mini", n) for n in (1, 9, 24, 32)),                    # [1, 2, 3, 4] 1 pass
+    *(("mini17", n) for n in (7, 16, 32)),                     # [1, 2, 4]
+    ("mini", 33), ("mini", 64), ("mini17", 33), ("mini17", 64),  # [5, 8] 2
+    *(("mini", n) for n in (65, 80, 100, 128)),                # [9, 10, 13, 16] 4
+    *(("mini17", n) for n in (41, 49)),                        # [6, 7] 2
+    *(("mini17", n) for n in (65, 96, 128)),                   # [9, 12, 16] 4
+    *(("mini", n) for n in (131, 160, 161, 192)),              # [17, 20, 21, 24] 6
+    *(("mini", n) for n in (193, 225, 256)),                   # [25, 29, 32] 8
+]
+# 128-row tiles, QKV split over K with qkv_post_kernel, O and down split over K, the attention in key-range
+# chunks; gate/up is never split from position 0 (a chunk of 97-128 tokens at 1.7B is: the 104 tokens at 196 of
+# test_prefill_in_chunks_and_decode_after_it).
+TILES_SPLIT = [("mini", 257), ("mini", 300), ("mini17", 129), ("mini17", 200)]
+# 256-row tiles: gate/up (three 128-row tiles in two at 300; 8 row tiles at 1,000), QKV too at 1,100 and at the
+# 1.7B 1,500. 656 tokens are the last on 128-row gate/up tiles, 657 the first on 256 rows.
+TILES_TALL = [("mini17_2k", 300), ("mini_4k", 656), ("mini_4k", 657), ("mini_4k", 1000), ("mini_4k", 1100)]
+# O and down unsplit, two wave groups halving K: 24 row tiles of 8 column tiles, 12 of 16
+TILES_LONG = [("mini_4k", 3000), ("mini17_2k", 1500)]
+
+
+@pytest.mark.parametrize("shape_fixture, P", SKINNY + TILES_SPLIT + TILES_TALL + TILES_LONG)
 def test_prefill_matches_oracle(shape_fixture, P, request):
     """Prefill from an empty cache against ``restate.prefill`` on the same prompt: the last token's
-    logits and greedy token, every K/V row written, and nothing written past the prompt. P = 1 has
-    one key; P <= 256 at the 0.6B width and P <= 128 at 1.7B run the skinny products on activations in
-    skinny fragment order, column blocks of 8 tokens (7: one, 9 and 16: two, 24 and 32: four, 33: five
-    of six in two workgroups, 192: 24 of six per workgroup), with the attention straight from the
-    products' sums in passes of 32 keys (1, 2, 4, 6 and 8 of them); P = 257 and the 1.7B P = 129 the
-    128-row tiles (rows past the prompt dead; QKV and gate/up split over K into raw sums that the post kernels
-    finish, the residual products split over K, several K steps in flight); P = 65 has two attention
-    query blocks, the second with one row; P = 300 spans 5 query blocks of the attention (key-range
-    chunks) and 3 row tiles of the products. From 8 row tiles the residual products are placed row tile by row tile on the
-    XCDs: P = 1000 (8 row tiles, 4-way K split), P = 3000 at the 0.6B width (24 row tiles, 192
-    tiles: no split, two wave groups halving K) and P = 1500 at the 1.7B width (12 row tiles of 16 column
-    tiles: the same). Grids between one and two workgroups per CU take 256-row tiles: gate/up at P = 1000
-    and the 1.7B P = 300 (three 128-row tiles in two), QKV at P = 1100;
-    not at most 16 rows past full tiles that leave CUs over: gate/up at P = 656, 256-row tiles at 657."""
+    logits and greedy token, every K/V row written, and nothing written past the prompt."""
     sess = request.getfixturevalue(shape_fixture)
     ids = hf.prompt_ids(P, sess.shape.vocab, seed=3)[0].tolist()
     s = sess.shape
@@ -112,13 +114,14 @@ def test_prefill_matches_oracle(shape_fixture, P, request):
                                                  ("mini_4k", (0, 1801, 2101))],
                          ids=["chunks-40-75", "chunks-900-964", "chunks-100-196-1.7b", "chunks-3-250", "chunks-1801"])
 def test_prefill_in_chunks_and_decode_after_it(shape_fixture, cuts, request):
-    """A prompt fed in three chunks gives the cache and last logits of the one-shot oracle prefill;
-    a decode step after it (the decode kernel, reading the prefilled cache) matches the oracle's
-    decode step on the oracle's cache. The chunks at 900 and 964 are short prompts (64 and 36
-    tokens) over 16 key blocks each (the 1.7B chunks: skinny products from position 0 and, of 96 tokens,
-    from 100, tiles for 104 tokens from 196; the 0.6B ones of 247 and 260 tokens the same): their attention runs as key-range chunks of two blocks on 64
-    workgroups, merged by attn_merge_kernel; the first chunk (900 tokens) as chunks of 5 key
-    blocks (of 4 a few short ones would run as a second round), the 300 tokens at 1,801 as chunks of 6."""
+    """A prompt fed in chunks gives the cache and last logits of the one-shot oracle prefill; a decode step
+    after it (the decode kernel, reading the prefilled cache) matches the oracle's decode step on the
+    oracle's cache. Chunks past position 0 on the skinny products with the general attention: 35 and 25
+    tokens (no key-range chunks), 64 at 900 and 36 at 964 (16 key blocks in chunks of two on 64
+    workgroups, merged by attn_merge_kernel), 247 at 3, and 96 at 100 at 1.7B. On tiles: 260 at 250, 300 at
+    1,801 (key-range chunks of 6 blocks), and 104 at 196 at 1.7B, the case whose gate/up product is split
+    over K (silu_post_kernel). The 900 tokens from position 0 take chunks of 5 key blocks (of 4 a few
+    short ones would run as a second round)."""
     mini = request.getfixturevalue(shape_fixture)
     P = cuts[-1]
     ids = hf.prompt_ids(P, mini.shape.vocab, seed=4)[0].tolist()
@@ -246,7 +249,14 @@ def _pool(sess, ps, extra, seed):
 
 
 @pytest.mark.parametrize("shape_fixture, chunks, ps", [
-    ("mini", ((0, 40),), 16),                      # short path
+    ("mini", ((0, 40),), 16),                      # skinny products, pages written by short_attn_kernel<2>
+    ("mini", ((0, 7),), 16),                       # ... <1>
+    ("mini", ((0, 100),), 16),                     # ... <4>
+    ("mini", ((0, 180),), 32),                     # ... <6>
+    ("mini", ((0, 250),), 16),                     # ... <8>
+    ("mini17", ((0, 100),), 16),                   # ... <4>, 1.7B width
+    ("mini", ((0, 3), (3, 250)), 16),              # skinny products past position 0: pages from qkv_post_kernel
+    ("mini17", ((0, 100), (100, 204)), 16),        # 1.7B tiles with gate/up split over K
     ("mini", ((0, 300),), 16),                     # 128-row tiles, residual products split over K
     ("mini17", ((0, 200),), 64),
     ("mini", ((0, 40), (40, 75), (75, 100)), 32),  # chunks reading earlier chunks through the table
@@ -291,21 +301,24 @@ def test_paged_prefill_matches_contiguous(shape_fixture, chunks, ps, request):
     assert sess.kernel.status() == 0
 
 
-def test_paged_prefill_bad_table_entry_is_reported_in_band(mini):
+@pytest.mark.parametrize("P, bad", [(40, 1), (250, 14), (300, 17)])
+def test_paged_prefill_bad_table_entry_is_reported_in_band(mini, P, bad):
     """A block-table entry outside the pool, on a page the prompt writes, cannot be checked on the host
     without a copy: the call reports NaN logits and token -1 and writes nothing through that entry."""
     s = mini.shape
     ps = 16
     table, kp, vp, pool = _pool(mini, ps, 2, 3)
-    table[1] = pool + 5  # positions 16..31
-    tokens = torch.tensor(hf.prompt_ids(40, s.vocab, seed=2)[0].tolist(), dtype=torch.int32, device=DEV)
-    before = kp.clone()
+    table[bad] = pool + 5  # positions 16 bad .. 16 bad + 15
+    tokens = torch.tensor(hf.prompt_ids(P, s.vocab, seed=2)[0].tolist(), dtype=torch.int32, device=DEV)
+    before = kp.clone()  # (vp holds the same)
     logits, tok = mini.kernel.prefill_paged(tokens, mini.embed, mini.lm_head, mini.final_norm, mini.layers, mini.cos,
                                             mini.sin, kp, vp, table.to(DEV), 0, mini.max_seq)
     assert torch.isnan(logits).all() and int(tok.item()) == -1
-    changed = (kp.float().nan_to_num(7.0) != before.float().nan_to_num(7.0)).any(-1).any(-1).any(-1).any(0)
-    assert set(changed.nonzero().flatten().tolist()) <= {int(table[0]), int(table[2])}  # pages of rows 0-15, 32-39
-    table[1] = sorted(set(range(pool)) - set(table.tolist()))[0]  # an unused page: the next call is healthy
+    good = {int(table[i]) for i in range((P + ps - 1) // ps) if i != bad}  # the prompt's other pages
+    for pages in (kp, vp):
+        changed = (pages.float().nan_to_num(7.0) != before.float().nan_to_num(7.0)).any(-1).any(-1).any(-1).any(0)
+        assert set(changed.nonzero().flatten().tolist()) <= good
+    table[bad] = sorted(set(range(pool)) - set(table.tolist()))[0]  # an unused page: the next call is healthy
     logits, tok = mini.kernel.prefill_paged(tokens, mini.embed, mini.lm_head, mini.final_norm, mini.layers, mini.cos,
                                             mini.sin, kp, vp, table.to(DEV), 0, mini.max_seq)
     assert torch.isfinite(logits).all() and int(tok.item()) >= 0
