@@ -2225,20 +2225,20 @@ static Layout layout(int H, int I, int M, bool small) {
   L.bytes = o;
   return L;
 }
-// Workspace for a call of up to M tokens at any position. A layout of more tokens can be the smaller one:
-// it has fewer K splits, or is of the other path. Between such steps (a path's longest prompt, a full row
-// tile while a residual product still splits) a layout grows with M, so the largest is the one of M or of
-// the last size before a step.
+// Workspace that a call of M tokens needs, at whichever position.
+static size_t call_bytes(int H, int I, int M) {
+  return std::max(layout(H, I, M, small_prompt(H, M, 0)).bytes, layout(H, I, M, small_prompt(H, M, 1)).bytes);
+}
+// Workspace for calls of up to M tokens. A layout of more tokens can be the smaller one: it has fewer K
+// splits, or is of the other path. Between such steps (a path's longest prompt, a full row tile while a
+// residual product still splits) a layout grows with M, so the largest is the one of M or of the last size
+// before a step.
 static size_t prefill_bytes(int H, int I, int M) {
-  size_t n = 0;
-  auto at = [&](int m) {
-    for (int position = 0; position < 2; ++position) n = std::max(n, layout(H, I, m, small_prompt(H, m, position)).bytes);
-  };
-  at(M);
+  size_t n = call_bytes(H, I, M);
   for (int position = 0; position < 2; ++position)
-    if (small_m(H, position) < M) at(small_m(H, position));
+    if (small_m(H, position) < M) n = std::max(n, call_bytes(H, I, small_m(H, position)));
   const int last = 192 / std::max(H / NT, 1);  // row tiles from which no product splits (resid_splits)
-  for (int t = 1; t <= last && t * MT < M; ++t) at(t * MT);
+  for (int t = 1; t <= last && t * MT < M; ++t) n = std::max(n, call_bytes(H, I, t * MT));
   return n;
 }
 static Work carve(void* base, const Layout& L) {
@@ -2441,9 +2441,9 @@ static hipError_t prefill_impl(const mk_model_dims* dims, const int32_t* tokens,
   if (!(s06 || s17) || dims->num_layers < 1 || dims->vocab < 1) return hipErrorInvalidValue;
   if (num_tokens < 1 || position < 0 || max_seq_len < 1 || (long long)position + num_tokens > max_seq_len)
     return hipErrorInvalidValue;
+  if (workspace_bytes < call_bytes(dims->hidden, dims->intermediate, num_tokens)) return hipErrorInvalidValue;
   const Layout L = layout(dims->hidden, dims->intermediate, num_tokens,
                           small_prompt(dims->hidden, num_tokens, position));
-  if (workspace_bytes < L.bytes) return hipErrorInvalidValue;
   const Work wk = carve(workspace, L);
   if (reinterpret_cast<uintptr_t>(workspace) % 256 != 0) return hipErrorInvalidValue;
   const mk_layer_weights* lw = static_cast<const mk_layer_weights*>(layer_weights);  // host array

@@ -253,6 +253,9 @@ def test_prefill_entry_point_rejects_bad_arguments_before_launch(lib):
     assert call(position=500, n=13) == HIP_ERROR_INVALID_VALUE  # past max_seq_len
     assert call(nbytes=n1 - 1) == HIP_ERROR_INVALID_VALUE
     assert call(workspace=vp(256 + 16)) == HIP_ERROR_INVALID_VALUE  # not 256-byte aligned
+    wide = Dims(2048, 6144, 28, 151936)
+    # 97-128 tokens at this width take a smaller layout from position 0, but the size is one for every position
+    assert call(wide, n=100, nbytes=ws(ctypes.byref(wide), 100) - 1) == HIP_ERROR_INVALID_VALUE
     assert call(workspace=None) == HIP_ERROR_INVALID_VALUE
 
 
